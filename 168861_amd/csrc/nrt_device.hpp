@@ -143,6 +143,14 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Workgroup barrier that orders LDS accesses only: global loads and stores in flight
+// are not waited for (__syncthreads waits for every one).
+__device__ __forceinline__ void lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Grid barrier for a persistent launch (all blocks co-resident). bar[0] counts
 // arrivals, bar[1] is the generation. The wait is bounded: after spin_limit
 // polls, or once another block raised *err, it sets *err and returns so that
