@@ -5,6 +5,7 @@
 // k steps) or one graph of k steps (explicit).
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -21,6 +22,17 @@ void implicit_batch_expand(int precision, const void* table, const void* work,
 void implicit_batch_launch(int precision, int krylov, int threads, const void* wgrec, int nwg,
                            hipStream_t s);
 size_t implicit_slot_work_bytes();
+bool implicit_resident(const nrt_handle* h);
+size_t resident_rec_bytes();
+void resident_slot_shape(nrt_handle* h, int* groups, int* T, size_t* lds);
+void resident_slot_fill(nrt_handle* h, long long a0, long long a1, int trace_elem,
+                        long long interval, double* trace, void* out);
+int resident_capacity(int device, int T, size_t lds);
+// implicit.hip: CUs of the device for workgroups that wait for each other, held until
+// the returned object is gone (waits for other launches of the process that hold them)
+std::shared_ptr<void> device_share(int device, int cus);
+void resident_batch_launch(const void* recs, const void* work, const int2* map, unsigned* ticket,
+                           int nwg, int T, size_t lds, hipStream_t s);
 void implicit_slot_work(void* out, long long done, long long steps, int vn);
 int implicit_batch_capacity(int precision, int krylov, int threads);
 void implicit_slot_stats(nrt_handle* h, int* status, int64_t* inner);
@@ -59,6 +71,14 @@ constexpr int64_t kImplicitBytesPerElem = 420;
 constexpr int64_t kExplicitBytesPerElem = 64;
 constexpr int64_t kAdmissionReserve = 512ll << 20;  // left free for the runtime
 
+// Resident slots of at most this many unit threads a workgroup (about 1,400 rows) run
+// in a launch of their own while they fill the device: a workgroup of the large ones'
+// size would leave two thirds of its waves idle.
+constexpr int kResSmallT = 192;
+struct ResStep {  // ResWork of resident_dev.hpp
+  long long done, steps;
+};
+
 struct Slot;
 }  // namespace
 int64_t batch_footprint(const nrt_batch* b, int N, int64_t num_steps, int64_t trace_every);
@@ -96,6 +116,18 @@ struct nrt_batch {
   long long g = 0;                           // batch steps done
   bool dirty = true;
   std::vector<int> order;  // slot ids in table order
+  // implicit: the slots whose tree solve is resident, by unit threads per workgroup
+  // (small ones apart), largest first; per launch their steps, the workgroups' (slot,
+  // group) map and a ticket, in one upload
+  struct ResClass {
+    std::vector<int> ids;
+    int T = 0, maxG = 0;  // most unit threads, most workgroups of a slot
+    size_t lds = 0, map_at = 0;
+    int nwg = 0;
+  };
+  ResClass res[2];
+  DBuf<uint8_t> rtable, rwork;
+  std::vector<uint8_t> rwork_h;
   DBuf<uint8_t> table;
   DBuf<int2> blk;
   int nblk = 0;
@@ -111,8 +143,9 @@ struct nrt_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   long long graph_k = 0;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
   bool pending = false;  // a launch is in flight (finish() accounts for it)
+  std::shared_ptr<void> share;  // CUs that its waiting workgroups need
   int64_t pend_cs = 0, pend_ss = 0, pend_launches = 0;
   int pend_threads = 0;
   // implicit: per size class, the workgroup size (0: still tuning), the tuning
@@ -169,6 +202,7 @@ struct nrt_batch {
       if (slots[id] && slots[id]->left() > 0) order.push_back(id);
     drop_graph();
     if (is_implicit()) {
+      rebuild_resident();
       // largest trees first: the long workgroups start early (LPT order)
       std::stable_sort(order.begin(), order.end(),
                        [&](int a, int b) { return slots[a]->N > slots[b]->N; });
@@ -202,6 +236,95 @@ struct nrt_batch {
     dirty = false;
   }
 
+  // Takes the slots with a resident tree solve out of `order`. Those of at most
+  // kResSmallT unit threads a workgroup get a launch of their own while they fill the
+  // device (as size classes do); else all share one.
+  void rebuild_resident() {
+    for (ResClass& c : res) c = ResClass();
+    std::vector<int> rest;
+    for (int id : order) {
+      if (!implicit_resident(slots[id]->h)) {
+        rest.push_back(id);
+        continue;
+      }
+      int G = 0, T = 0;
+      size_t lds = 0;
+      resident_slot_shape(slots[id]->h, &G, &T, &lds);
+      ResClass& c = res[T <= kResSmallT ? 1 : 0];
+      c.ids.push_back(id);
+      c.T = std::max(c.T, T);
+      c.lds = std::max(c.lds, lds);
+      c.maxG = std::max(c.maxG, G);
+    }
+    order.swap(rest);
+    if (!res[0].ids.empty() && !res[1].ids.empty() &&
+        (int)res[1].ids.size() < resident_capacity(device, res[1].T, res[1].lds) / 2) {
+      res[0].ids.insert(res[0].ids.end(), res[1].ids.begin(), res[1].ids.end());
+      res[0].lds = std::max(res[0].lds, res[1].lds);
+      res[0].maxG = std::max(res[0].maxG, res[1].maxG);
+      res[1] = ResClass();
+    }
+    const size_t rb = resident_rec_bytes();
+    std::vector<uint8_t> host;
+    for (ResClass& c : res) {
+      std::stable_sort(c.ids.begin(), c.ids.end(),
+                       [&](int a, int b) { return slots[a]->N > slots[b]->N; });
+      for (int id : c.ids) {
+        Slot& s = *slots[id];
+        host.resize(host.size() + rb);
+        resident_slot_fill(s.h, s.a0, s.a1, s.trace_elem, s.interval, s.trace.p,
+                           host.data() + host.size() - rb);
+      }
+    }
+    rtable.upload(host, stream);
+    NRT_HIP(hipStreamSynchronize(stream));
+  }
+
+  // Enqueues the resident slots' steps (largest workgroups first).
+  void launch_resident(long long k, long long elem_budget, long long kmax, int64_t& cs,
+                       int64_t& ss) {
+    const size_t n = res[0].ids.size() + res[1].ids.size();
+    if (n == 0) return;
+    std::vector<int2> map;
+    rwork_h.assign(n * sizeof(ResStep), 0);
+    size_t at = 0;
+    for (ResClass& c : res) {
+      c.map_at = map.size();
+      for (int id : c.ids) {
+        Slot& s = *slots[id];
+        int G = 0, T = 0;
+        size_t lds = 0;
+        resident_slot_shape(s.h, &G, &T, &lds);
+        long long want = k;
+        if (elem_budget > 0)
+          want = std::max(1ll, std::min(kmax > 0 ? kmax : k, elem_budget * G / std::max(1, s.N)));
+        const ResStep w{s.done, std::min(want, s.left())};
+        memcpy(rwork_h.data() + at * sizeof(ResStep), &w, sizeof(w));
+        if (w.steps > 0)
+          for (int g = 0; g < G; g++) map.push_back(make_int2((int)at, g));
+        s.done += w.steps;
+        ss += w.steps;
+        cs += w.steps * s.N;
+        at++;
+      }
+      c.nwg = (int)(map.size() - c.map_at);
+    }
+    // steps, map, tickets
+    const size_t map_at = rwork_h.size(), tick_at = map_at + map.size() * sizeof(int2);
+    rwork_h.resize(tick_at + 2 * sizeof(int2), 0);
+    memcpy(rwork_h.data() + map_at, map.data(), map.size() * sizeof(int2));
+    if (rwork.n < rwork_h.size()) rwork.alloc(2 * rwork_h.size());
+    NRT_HIP(hipMemcpyAsync(rwork.p, rwork_h.data(), rwork_h.size(), hipMemcpyHostToDevice, stream));
+    for (int c = 0; c < 2; c++) {
+      if (res[c].nwg == 0) continue;
+      resident_batch_launch(rtable.p, rwork.p, (const int2*)(rwork.p + map_at) + res[c].map_at,
+                            (unsigned*)(rwork.p + tick_at) + 2 * c, res[c].nwg, res[c].T,
+                            res[c].lds, stream);
+      pend_launches++;
+    }
+  }
+  bool any_resident() const { return !res[0].ids.empty() || !res[1].ids.empty(); }
+
   int pick_threads(int c) {
     if (opt.batch_threads > 0) return opt.batch_threads;
     if (cthreads[c] > 0) return cthreads[c];
@@ -219,7 +342,27 @@ struct nrt_batch {
                 "explicit batches step in lockstep");
     if (dirty) rebuild();
     g += k;
-    if (order.empty() || k == 0) return;
+    if ((order.empty() && !any_resident()) || k == 0) return;
+    int64_t cs = 0, ss = 0, ccs[kClasses] = {0, 0, 0};
+    pend_launches = 0;
+    std::shared_ptr<void> held;  // (given back at once if the launch fails)
+    if (any_resident()) {
+      // (the ticket leaves at most one neurite's workgroups waiting for others to start)
+      int most = 0;
+      for (const ResClass& c : res) most = std::max(most, c.maxG);
+      held = device_share(device, order.empty() ? most : INT_MAX);
+      NRT_HIP(hipEventRecord(ev0, stream));
+      launch_resident(k, elem_budget, kmax, cs, ss);
+      if (order.empty()) {
+        for (ClassLaunch& c : pend_cls) c.on = false;
+        NRT_HIP(hipEventRecord(ev1, stream));
+        pend_cs = cs;
+        pend_ss = ss;
+        share = std::move(held);
+        pending = true;
+        return;
+      }
+    }
     int th[kClasses] = {0, 0, 0};
     std::vector<int2> seg;  // wgmap range of each class
     bool merged = false;    // one launch for all classes
@@ -243,7 +386,6 @@ struct nrt_batch {
         seg = plan_workgroups(th);
       }
     }
-    int64_t cs = 0, ss = 0, ccs[kClasses] = {0, 0, 0};
     const size_t wb = implicit_slot_work_bytes();
     for (size_t i = 0; i < order.size(); i++) {
       Slot& s = *slots[order[i]];
@@ -273,9 +415,16 @@ struct nrt_batch {
       // back, so that no launch waits for another's tail. A slot spanning several
       // workgroups still finds them all resident: its launch alone fits the
       // co-resident limit, and the other launches' workgroups wait on nothing.
-      pend_launches = 0;
+      int waiting = 0;  // workgroups of a launch with virtual grids
+      for (size_t i = 0; i < order.size(); i++)
+        if (vn[i] > 1) waiting = nwg;
+      if (waiting > 1 && !held) held = device_share(device, waiting);
+      // (after the resident slots' launch on the same stream: workgroups that wait for
+      // each other are never resident beside another such launch's)
       int64_t best = -1;
-      NRT_HIP(hipEventRecord(ev0, stream));
+      if (!any_resident()) NRT_HIP(hipEventRecord(ev0, stream));
+      hipEvent_t fork = any_resident() ? ev2 : ev0;
+      if (any_resident()) NRT_HIP(hipEventRecord(ev2, stream));
       hipStream_t on = nullptr;
       if (merged) {  // the whole wgmap as the dominant class's launch
         seg.assign(kClasses, make_int2(0, 0));
@@ -291,7 +440,7 @@ struct nrt_batch {
         const int n = seg[c].y - seg[c].x;
         if (n <= 0) continue;
         const hipStream_t cs_ = on == nullptr ? stream : side[c];
-        if (cs_ != stream) NRT_HIP(hipStreamWaitEvent(cs_, ev0, 0));
+        if (cs_ != stream) NRT_HIP(hipStreamWaitEvent(cs_, fork, 0));
         on = cs_;
         NRT_HIP(hipEventRecord(cev[c][0], cs_));
         implicit_batch_launch(opt.precision, opt.krylov, th[c], wgrec.p + rec1 * seg[c].x, n,
@@ -328,6 +477,7 @@ struct nrt_batch {
     }
     pend_cs = cs;
     pend_ss = ss;
+    share = std::move(held);
     pending = true;
   }
 
@@ -383,6 +533,7 @@ struct nrt_batch {
   void finish() {
     if (!pending) return;
     pending = false;
+    const auto held = std::move(share);  // given back at the end
     float ms = 0;
     if (is_implicit()) {
       NRT_HIP(hipEventSynchronize(ev1));
@@ -414,6 +565,9 @@ struct nrt_batch {
     stats.compartment_steps += pend_cs;
     for (int id : order)
       if (slots[id] && slots[id]->left() <= 0) dirty = true;
+    for (ResClass& c : res)
+      for (int id : c.ids)
+        if (slots[id] && slots[id]->left() <= 0) dirty = true;
   }
 
   void step(long long k) {
@@ -464,6 +618,7 @@ int nrt_batch_create(const nrt_options* opt, nrt_batch** out) {
     NRT_HIP(hipStreamCreateWithFlags(&b->adm, hipStreamNonBlocking));
     NRT_HIP(hipEventCreate(&b->ev0));
     NRT_HIP(hipEventCreate(&b->ev1));
+    NRT_HIP(hipEventCreate(&b->ev2));
     for (int c = 0; c < kClasses; c++) {
       for (int e = 0; e < 2; e++) NRT_HIP(hipEventCreate(&b->cev[c][e]));
       if (b->opt.kind == NRT_IMPLICIT && c < kClasses - 1)
@@ -762,6 +917,7 @@ int nrt_batch_destroy(nrt_batch* b) {
   }
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
+  if (b->ev2) (void)hipEventDestroy(b->ev2);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   if (b->adm) (void)hipStreamDestroy(b->adm);
   delete b;
@@ -817,7 +973,10 @@ int batch_add_handle(nrt_batch* b, nrt_handle* h, int64_t num_steps, int64_t a0,
 }
 
 static bool in_flight(const nrt_batch* b, int slot) {
-  return b->pending && std::find(b->order.begin(), b->order.end(), slot) != b->order.end();
+  if (!b->pending) return false;
+  for (const auto& c : b->res)
+    if (std::find(c.ids.begin(), c.ids.end(), slot) != c.ids.end()) return true;
+  return std::find(b->order.begin(), b->order.end(), slot) != b->order.end();
 }
 
 void batch_slot_collect(nrt_batch* b, int slot, hipStream_t side, std::vector<double>* V,

@@ -24,15 +24,19 @@
 // rowptr/col (int32), val; per element cmdx = c_m*dx, kdx = K*dx, rdx = r_a*dx,
 // input, code (uint32); HH SoA as in the explicit step plus row type/position/DL.
 #include <algorithm>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <numeric>
+#include <thread>
 #include <tuple>
 #include <type_traits>
 #include "nrt_internal.hpp"
 #include "nrt_device.hpp"
-#include "implicit_dev.hpp"
+#include "resident_dev.hpp"
 #include "tree.hpp"
 
 namespace nrt {
@@ -42,6 +46,10 @@ bool krylov_block_ok(int N, bool gmres, bool mixed, int restart, int max_lds);
 void krylov_block_prepare(int N, bool gmres, int m);
 void bicgstab_block_launch(ImpDev d, hipStream_t s);
 void gmres_block_launch(ImpDev d, GmresDev<double> g, hipStream_t s);
+// resident.hip
+size_t resident_lds(const ResDev& r);
+int resident_capacity(int device, int T, size_t lds);
+void resident_launch(const ImpDev& d, const ResDev& r, const ResRun& q, hipStream_t s);
 
 struct Implicit {
   int N = 0, H = 0, nnz = 0, nblocks = 0;
@@ -85,6 +93,17 @@ struct Implicit {
   TreePlanDev plan{};
   DBuf<double> tw64, tw64alt;  // alt: the second top-input buffer (group-resident form)
   DBuf<float> tw32, tw32alt;
+  // tree solve with resident rows (resident.hpp)
+  bool resident = false;
+  ResDev rdev{};
+  DBuf<double> rx2, rcdt, rkd, rinp, rF, rI, ruco, rpz, rtop, rdyn;
+  DBuf<uint32_t> ruinf;
+  DBuf<uint16_t> rinf16;
+  DBuf<int32_t> rinf32;
+  DBuf<unsigned long long> rll;
+  unsigned rtag = 0;  // tag of the last step launched
+  int64_t rsteps = 0;
+  std::vector<int32_t> rslot;  // element -> index in x
 };
 
 // ------------------------------------------------------------------ assembly
@@ -2039,6 +2058,156 @@ static int choose_blocks(nrt_handle* hnd, int N, const void* kernel = nullptr) {
   return std::max(1, want);
 }
 
+// The resident form (resident.hpp) of a FP64 direct solve, with every option that
+// shapes the other forms left to the library. Taken whenever its plan exists and a
+// launch's workgroups are all resident at once, whatever the size: per step, 700 rows
+// 30.4 us in block form, 2.7 resident; 3,001 rows 36.7 and 4.3; 60,000 rows (17 groups)
+// 49.7 (local form) and 9.5; 902,037 rows (255 groups) 120 and 14.0.
+static bool resident_create(nrt_handle* hnd, Implicit* e, const HostProblem& p,
+                            const std::vector<int32_t>& par, const std::vector<int32_t>& rowptr,
+                            const std::vector<int32_t>& col, const std::vector<double>& cmdx,
+                            const std::vector<double>& kdx, bool in_batch) {
+  const nrt_options& o = hnd->opt;
+  const int N = e->N, H = e->H;
+  hipStream_t s = hnd->stream;
+  if (o.num_blocks != 0 || o.chunk != 0 || o.chunk_hi != 0 || o.tree_groups != 0 ||
+      o.batch_threads != 0 || H > kResDyn)
+    return false;
+  std::vector<double> val(e->nnz);
+  std::vector<int32_t> type(H);
+  NRT_HIP(hipMemcpyAsync(val.data(), e->val.p, sizeof(double) * e->nnz, hipMemcpyDeviceToHost, s));
+  if (H > 0)
+    NRT_HIP(hipMemcpyAsync(type.data(), e->hh_type.p, sizeof(int32_t) * H, hipMemcpyDeviceToHost,
+                           s));
+  NRT_HIP(hipStreamSynchronize(s));
+  for (int hh = 0; hh < H; hh++)  // an HH ghost or sealed end gates without a row of its own
+    if (type[hh] == RT_OTHER || type[hh] == RT_TERM) return false;
+  std::vector<double> diag(N, 0.0), up(N, 0.0), dn(N, 0.0);
+  for (int i = 0; i < N; i++)
+    for (int k = rowptr[i]; k < rowptr[i + 1]; k++) {
+      if (col[k] == i) diag[i] = val[k];
+      else if (col[k] < i) up[i] = val[k];
+      else dn[col[k]] = val[k];
+    }
+  ResPlanHost P;
+  std::string why;
+  // lanes of a group: the units a small tree needs (estimated), else kResT
+  const int units = N / kResC + N / 32 + 8;
+  const int T = units <= kResT ? std::max(kWave, grid_for(units, kWave) * kWave) : kResT;
+  const std::vector<int32_t> hh_row(p.hh_elem.begin(), p.hh_elem.end());
+  if (!build_resident_plan(N, par, diag, up, dn, hh_row, T, P, why)) return false;
+  ResDev& r = e->rdev;
+  r = ResDev{};
+  r.G = P.G;
+  r.T = P.T;
+  r.nd = P.nd;
+  r.nt = P.nt;
+  r.npub = P.npub;
+  r.nth = P.nth;
+  r.top_narrow = P.top_narrow;
+  r.rounds = P.rounds;
+  r.owner = P.owner;
+  const size_t lds = resident_lds(r);
+  int max_lds = 0;
+  NRT_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, hnd->device));
+  if (lds + 1024 > (size_t)max_lds || P.G > resident_capacity(hnd->device, P.T, lds)) return false;
+  // rows in slot order
+  const size_t n0 = (size_t)P.ns0();
+  std::vector<double> x(n0, 0.0), cdt(n0, 0.0), kd(n0, 0.0), inp;
+  for (int i = 0; i < N; i++) {
+    const size_t at = (size_t)P.slot[i];
+    x[at] = p.V0[i];
+    cdt[at] = cmdx[i] / p.dT;
+    kd[at] = kdx[i];
+    if (p.input[i] != 0.0 && at < n0 - 4 * P.nd) {
+      if (inp.empty()) inp.assign(n0, 0.0);
+      inp[at] = p.input[i];
+    }
+  }
+  for (int j = 0; j < P.nd; j++)
+    for (int k = 0; k < H; k++)
+      if (p.hh_elem[k] == P.dyn_row[j]) {
+        double* at = x.data() + (n0 - 4 * P.nd) + j;
+        at[P.nd] = p.m[k];
+        at[2 * P.nd] = p.h[k];
+        at[3 * P.nd] = p.n[k];
+      }
+  e->x.upload(x, s);
+  if (!in_batch && P.G > 1) e->rx2.upload(x, s);
+  e->rcdt.upload(cdt, s);
+  e->rkd.upload(kd, s);
+  if (!inp.empty()) e->rinp.upload(inp, s);
+  e->rF.upload(P.F, s);
+  e->rI.upload(P.I, s);
+  e->ruco.upload(P.uco, s);
+  e->rpz.upload(P.pz, s);
+  e->ruinf.upload(P.uinf, s);
+  std::vector<double> top(P.tz), dyn;
+  top.insert(top.end(), P.te.begin(), P.te.end());
+  e->rtop.upload(top, s);
+  std::vector<uint16_t> u16(P.pinf);
+  const size_t at_t = u16.size();
+  u16.insert(u16.end(), P.tinf.begin(), P.tinf.end());
+  const size_t at_d = u16.size();
+  u16.insert(u16.end(), P.dinf.begin(), P.dinf.end());
+  const size_t at_e = u16.size();
+  u16.insert(u16.end(), P.epiece.begin(), P.epiece.end());
+  e->rinf16.upload(u16, s);
+  std::vector<int32_t> i32(P.ginfo);
+  const size_t at_h = i32.size();
+  i32.insert(i32.end(), P.thoff.begin(), P.thoff.end());
+  const size_t at_r = i32.size();
+  for (int j = 0; j < P.nd; j++) i32.push_back(P.dyn_row[j]);
+  const size_t at_hh = i32.size();
+  for (int j = 0; j < P.nd; j++) {
+    int hh = -1;
+    for (int k = 0; k < H; k++)
+      if (p.hh_elem[k] == P.dyn_row[j]) hh = k;
+    i32.push_back(hh);
+    dyn.push_back(diag[P.dyn_row[j]]);
+  }
+  e->rinf32.upload(i32, s);
+  dyn.insert(dyn.end(), P.dyn_s.begin(), P.dyn_s.end());
+  dyn.insert(dyn.end(), P.dyn_u.begin(), P.dyn_u.end());
+  e->rdyn.upload(dyn, s);
+  e->rll.alloc(4 * (size_t)P.npub);
+  NRT_HIP(hipMemsetAsync(e->rll.p, 0, sizeof(unsigned long long) * 4 * P.npub, s));
+  r.has_input = inp.empty() ? 0 : 1;
+  r.cdt = e->rcdt.p;
+  r.kd = e->rkd.p;
+  r.inp = e->rinp.p;
+  r.F = e->rF.p;
+  r.I = e->rI.p;
+  r.x = e->x.p;
+  r.xo = e->rx2.p ? e->rx2.p : e->x.p;
+  r.uco = e->ruco.p;
+  r.uinf = e->ruinf.p;
+  r.pz = e->rpz.p;
+  r.pinf = e->rinf16.p;
+  r.tinf = e->rinf16.p + at_t;
+  r.dinf = e->rinf16.p + at_d;
+  r.epiece = e->rinf16.p + at_e;
+  r.ginfo = e->rinf32.p;
+  r.thoff = e->rinf32.p + at_h;
+  r.drow = e->rinf32.p + at_r;
+  r.dhh = e->rinf32.p + at_hh;
+  r.tz = e->rtop.p;
+  r.te = e->rtop.p + P.nt;
+  r.ddiag = e->rdyn.p;
+  r.ds = e->rdyn.p + P.nd;
+  r.du = e->rdyn.p + 2 * P.nd;
+  r.ll = e->rll.p;
+  NRT_HIP(hipStreamSynchronize(s));  // the host arrays end here
+  e->resident = true;
+  e->rslot = std::move(P.slot);
+  e->ns0 = (int)n0;
+  e->nblocks = P.G;
+  e->threads = P.T;
+  e->rowptr.release();
+  e->col.release();
+  return true;
+}
+
 Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threads) {
   hipStream_t s = hnd->stream;
   const int N = p.N, H = p.H;
@@ -2172,6 +2341,9 @@ Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threa
           NRT_REQUIRE(hcol[k] <= i || par[hcol[k]] == i, NRT_ERR_TOPOLOGY,
                       "tree solve: row " + std::to_string(i) + " couples to row " +
                           std::to_string(hcol[k]) + ", which does not couple back");
+      if (e->method == 1 && resident_create(hnd, e, p, par, hrp, hcol, cmdx, kdx, batch_threads > 0)) {
+        // (everything is set up: rows, plan, launch form)
+      } else {
       // Workgroups: every reduction level costs a grid barrier (an L2 write-back), so
       // a mid-size tree runs best in one workgroup (measured on a 20,202-row cable
       // with reused factors: 1 -> 71 us, 4 -> 81 us per step) and only large trees
@@ -2400,6 +2572,7 @@ Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threa
           NRT_HIP(hipMemsetAsync(e->tw32alt.p, 0, sizeof(float) * kTreeArrays * T, s));
         }
       }
+      }
     } else if (o.krylov == NRT_GMRES) {
       e->gmres = true;
       e->gm = std::min(o.restart, N);
@@ -2510,7 +2683,7 @@ static ImpDev imp_dev(nrt_handle* hnd) {
 // level-0 slot for the tree solve.
 static int32_t probe_index(const Implicit* e, int32_t elem, int64_t interval) {
   if (interval < 0 || elem < 0 || elem >= e->N) return 0;  // no probe: never read
-  return e->method != 0 ? e->plan_h.slot0[elem] : elem;
+  return e->method == 0 ? elem : e->resident ? e->rslot[elem] : e->plan_h.slot0[elem];
 }
 
 template <class T>
@@ -2549,7 +2722,7 @@ static TreeArgs<T> tree_args(Implicit* e, const nrt_options& o, T* b, T* alt = n
 // test run, two simulations) would be refused its launches.
 static int launch_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64_t a1,
                              int32_t trace_elem, int64_t interval, double* trace_dev,
-                             int64_t gl0 = 0) {
+                             int64_t gl0 = 0, bool retried = false) {
   Implicit* e = hnd->im;
   const nrt_options& o = hnd->opt;
   ImpDev d = imp_dev(hnd);
@@ -2593,6 +2766,15 @@ static int launch_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_
                                        dim3(kImpBlock), args, 0, hnd->stream));
     return NRT_OK;
   }
+  if (e->resident) {
+    // the first exchange waits for workgroups that have not started: about 20 ms where
+    // the caller tries again (run_persistent), later ones only for each other
+    const ResRun q{first, num, gl0, e->rtag, trace_dev,
+                   retried ? std::min(d.spin_limit, 20000ull) : d.spin_limit};
+    e->rtag += (unsigned)num;
+    resident_launch(d, e->rdev, q, hnd->stream);
+    return NRT_OK;
+  }
   auto launch = [&](auto targs, const void* kgrid, const void* kblock, const void* klocal) {
     void* args[] = {&d, &targs};
     using TT = typename std::remove_pointer<decltype(targs.w.d)>::type;
@@ -2618,6 +2800,54 @@ static int launch_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_
            (const void*)(e->local_res ? (const void*)k_implicit_tree_local<float, true>
                                       : (const void*)k_implicit_tree_local<float, false>));
   return NRT_OK;
+}
+
+// Workgroups that wait for each other must all be resident at once. Launches of one
+// process on one device take their number of CUs here, in order of asking, and give it
+// back when they have ended, so two such launches on different streams never hold parts
+// of the device that the other one needs.
+class DeviceShare {
+ public:
+  DeviceShare(int device, int cus_wanted) : device_(device) {
+    if (cus_wanted <= 1) return;
+    Pool& p = pool(device);
+    std::unique_lock<std::mutex> g(p.mu);
+    if (p.total == 0)
+      NRT_HIP(hipDeviceGetAttribute(&p.total, hipDeviceAttributeMultiprocessorCount, device));
+    n_ = std::min(cus_wanted, p.total);
+    const unsigned long long mine = p.next++;
+    p.cv.wait(g, [&] { return p.serving == mine && p.used + n_ <= p.total; });
+    p.serving++;
+    p.used += n_;
+    p.cv.notify_all();
+  }
+  DeviceShare(const DeviceShare&) = delete;
+  DeviceShare& operator=(const DeviceShare&) = delete;
+  ~DeviceShare() {
+    if (n_ == 0) return;
+    Pool& p = pool(device_);
+    std::lock_guard<std::mutex> g(p.mu);
+    p.used -= n_;
+    p.cv.notify_all();
+  }
+
+ private:
+  struct Pool {
+    std::mutex mu;
+    std::condition_variable cv;
+    unsigned long long next = 0, serving = 0;
+    int used = 0, total = 0;
+  };
+  static Pool& pool(int device) {
+    static std::mutex mu;
+    static std::map<int, Pool> pools;
+    std::lock_guard<std::mutex> g(mu);
+    return pools[device];
+  }
+  int device_, n_ = 0;
+};
+std::shared_ptr<void> device_share(int device, int cus) {
+  return cus <= 1 ? nullptr : std::shared_ptr<void>(std::make_shared<DeviceShare>(device, cus));
 }
 
 // Zero the grid barrier's words (arrivals, generation, error flag) after a launch
@@ -2672,8 +2902,8 @@ static int collect_stats(nrt_handle* hnd) {
   NRT_HIP(hipMemcpyAsync(&st, e->st.p, sizeof(ImpStats), hipMemcpyDeviceToHost, hnd->stream));
   NRT_HIP(hipMemcpyAsync(&err, e->bar.p + 2, sizeof(unsigned), hipMemcpyDeviceToHost, hnd->stream));
   NRT_HIP(hipStreamSynchronize(hnd->stream));
-  hnd->stats.steps = (int64_t)st.steps;
-  hnd->stats.krylov_iters = (int64_t)st.iters_total;
+  hnd->stats.steps = e->resident ? e->rsteps : (int64_t)st.steps;
+  hnd->stats.krylov_iters = e->resident ? e->rsteps : (int64_t)st.iters_total;
   hnd->stats.refine_sweeps =
       hnd->opt.precision == NRT_FP32_REFINE || e->method >= 3 ? (int64_t)st.sweeps_total : 0;
   hnd->stats.last_iters = st.last_iters;
@@ -2683,6 +2913,7 @@ static int collect_stats(nrt_handle* hnd) {
   hnd->stats.matrix_nnz = e->nnz;
   hnd->stats.num_blocks = e->nblocks;
   hnd->stats.tree_form = e->method == 0      ? -1
+                         : e->resident       ? NRT_TREE_RESIDENT
                          : e->local_mode     ? (e->local_res ? NRT_TREE_LOCAL_LDS : NRT_TREE_LOCAL)
                          : e->grid_mode      ? NRT_TREE_GRID
                                              : NRT_TREE_BLOCK;
@@ -2709,10 +2940,54 @@ static int collect_stats(nrt_handle* hnd) {
 
 void implicit_update(nrt_handle* hnd, bool active) { hnd->input_active = active; }
 
+// launch_persistent and its end. A resident launch whose workgroups did not all start
+// in time (another process holds part of the device) has left the state as it was: it is
+// tried again for as long as a wait inside the kernel would last, then reported.
+static void resident_flip(Implicit* e, int64_t num) {
+  e->rsteps += num;
+  if (!e->rx2.p) return;
+  std::swap(e->x.p, e->rx2.p);
+  e->rdev.x = e->x.p;
+  e->rdev.xo = e->rx2.p;
+}
+static void run_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64_t a1,
+                           int32_t trace_elem, int64_t interval, double* trace_dev,
+                           hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr) {
+  Implicit* e = hnd->im;
+  const auto share = device_share(hnd->device, e->nblocks);
+  const bool limited = getenv("NRT_SPIN_LIMIT") != nullptr;
+  const auto until = std::chrono::steady_clock::now() + std::chrono::seconds(limited ? 1 : 180);
+  for (int attempt = 0;; attempt++) {
+    if (t0) NRT_HIP(hipEventRecord(t0, hnd->stream));
+    launch_persistent(hnd, first, num, a0, a1, trace_elem, interval, trace_dev, 0, true);
+    if (t1) NRT_HIP(hipEventRecord(t1, hnd->stream));
+    if (!e->resident) {
+      if (share) NRT_HIP(hipStreamSynchronize(hnd->stream));
+      return;
+    }
+    if (e->rdev.G > 1) {
+      unsigned err = 0;
+      NRT_HIP(hipMemcpyAsync(&err, e->bar.p + 2, sizeof(unsigned), hipMemcpyDeviceToHost,
+                             hnd->stream));
+      NRT_HIP(hipStreamSynchronize(hnd->stream));
+      if (err && std::chrono::steady_clock::now() < until) {
+        reset_barrier(e, hnd->stream);
+        // (handles of different processes wait differently: their addresses differ)
+        std::this_thread::sleep_for(std::chrono::microseconds(
+            100 * std::min(attempt + 1, 50) + (int)((uint32_t)((uintptr_t)e >> 6) * 2654435761u >> 22)));
+        continue;
+      }
+      if (err) return;  // collect_stats reports it
+    }
+    resident_flip(e, num);
+    return;
+  }
+}
+
 int implicit_calculate(nrt_handle* hnd) {
   Implicit* e = hnd->im;
   const int64_t st = e->step;
-  launch_persistent(hnd, st, 1, hnd->input_active ? st : st + 1, st, 0, -1, nullptr);
+  run_persistent(hnd, st, 1, hnd->input_active ? st : st + 1, st, 0, -1, nullptr);
   e->step++;
   return collect_stats(hnd);
 }
@@ -2729,7 +3004,7 @@ void implicit_snapshot_on(nrt_handle* hnd, double* host_out, hipStream_t s) {
   std::vector<double> xs(e->ns0);  // slot order -> element order
   NRT_HIP(hipMemcpyAsync(xs.data(), e->x.p, sizeof(double) * e->ns0, hipMemcpyDeviceToHost, s));
   NRT_HIP(hipStreamSynchronize(s));
-  const int32_t* s0 = e->plan_h.slot0.data();
+  const int32_t* s0 = e->resident ? e->rslot.data() : e->plan_h.slot0.data();
   for (int i = 0; i < e->N; i++) host_out[i] = xs[s0[i]];
 }
 
@@ -2749,10 +3024,8 @@ int implicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64_
   hipEvent_t t0, t1;
   NRT_HIP(hipEventCreate(&t0));
   NRT_HIP(hipEventCreate(&t1));
-  NRT_HIP(hipEventRecord(t0, hnd->stream));
-  launch_persistent(hnd, first, num, a0, a1, trace_elem, interval,
-                    (tracing && trace_out) ? e->trace.p : nullptr);
-  NRT_HIP(hipEventRecord(t1, hnd->stream));
+  run_persistent(hnd, first, num, a0, a1, trace_elem, interval,
+                 (tracing && trace_out) ? e->trace.p : nullptr, t0, t1);
   const int64_t k = max_samples;
   if (trace_out && k > 0)
     NRT_HIP(hipMemcpyAsync(trace_out, e->trace.p, sizeof(double) * k, hipMemcpyDeviceToHost,
@@ -2778,7 +3051,8 @@ size_t implicit_slot_bytes(int precision) {
 void implicit_slot_fill(nrt_handle* h, long long a0, long long a1, int trace_elem,
                         long long interval, double* trace, void* out) {
   Implicit* e = h->im;
-  NRT_REQUIRE(e->method != 0 && !e->grid_mode && !e->local_mode, NRT_ERR_UNSUPPORTED,
+  NRT_REQUIRE(e->method != 0 && !e->grid_mode && !e->local_mode && !e->resident,
+              NRT_ERR_UNSUPPORTED,
               "batch slots use the block-mode tree solve");
   ImpDev d = imp_dev(h);
   d.a0 = a0;
@@ -2792,6 +3066,25 @@ void implicit_slot_fill(nrt_handle* h, long long a0, long long a1, int trace_ele
     BatchSlot<float> S{d, tree_args<float>(e, h->opt, e->tw32.p), trace};
     std::memcpy(out, &S, sizeof(S));
   }
+}
+
+// Slots whose tree solve is resident (resident.hip).
+bool implicit_resident(const nrt_handle* h) { return h->im && h->im->resident; }
+size_t resident_rec_bytes() { return sizeof(ResRec); }
+void resident_slot_shape(nrt_handle* h, int* groups, int* T, size_t* lds) {
+  *groups = h->im->rdev.G;
+  *T = h->im->rdev.T;
+  *lds = resident_lds(h->im->rdev);
+}
+void resident_slot_fill(nrt_handle* h, long long a0, long long a1, int trace_elem,
+                        long long interval, double* trace, void* out) {
+  ImpDev d = imp_dev(h);
+  d.a0 = a0;
+  d.a1 = a1;
+  d.interval = interval;
+  d.trace_elem = probe_index(h->im, trace_elem, interval);
+  const ResRec R{d, h->im->rdev, trace};
+  std::memcpy(out, &R, sizeof(R));
 }
 
 size_t implicit_slot_work_bytes() { return sizeof(SlotWork); }
@@ -2908,6 +3201,7 @@ void implicit_batch_launch(int precision, int krylov, int threads, const void* w
 void implicit_steps_async(nrt_handle* h, int64_t first, int64_t num, int64_t a0, int64_t a1,
                           int32_t trace_elem, int64_t interval, int64_t gl0, double* trace_dev) {
   launch_persistent(h, first, num, a0, a1, trace_elem, interval, trace_dev, gl0);
+  if (h->im->resident) resident_flip(h->im, num);
   h->im->step = first + num;
 }
 
@@ -2933,7 +3227,10 @@ int64_t implicit_device_bytes(const Implicit* e) {
   return N * (8 * 5 + 4) + S * (8 * 5 + 4) + (int64_t)e->nnz * 13 + (S + 1) * 4 +
          (int64_t)e->H * 8 * 13 + (int64_t)e->plan_buf.n * 4 +
          T * kTreeArrays * (e->method == 1 || e->method == 3 ? 8 : 4) +
-         (e->method >= 3 ? S * 8 * 8 : 0);
+         (e->method >= 3 ? S * 8 * 8 : 0) +
+         (e->resident ? (int64_t)(e->rF.n * 8 * 5 + e->ruco.n * 8 + e->ruinf.n * 4 + e->rpz.n * 8 +
+                                  e->rinf16.n * 2 + e->rll.n * 8)
+                      : 0);
 }
 
 }  // namespace nrt

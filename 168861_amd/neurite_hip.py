@@ -24,11 +24,12 @@ BICGSTAB, GMRES, DIRECT = 0, 1, 2
 PRECOND_NONE, PRECOND_TREE = 0, 1
 TOL_ABSOLUTE, TOL_RELATIVE = 0, 1
 X0_PREVIOUS, X0_RHS, X0_ZERO = 0, 1, 2
-TREE_BLOCK, TREE_GRID, TREE_LOCAL, TREE_LOCAL_LDS = 0, 1, 2, 3
+TREE_BLOCK, TREE_GRID, TREE_LOCAL, TREE_LOCAL_LDS, TREE_RESIDENT = 0, 1, 2, 3, 4
 # demangled name of the tree-solve kernel of each launch form (nrt_stats.tree_form)
 TREE_KERNELS = {TREE_BLOCK: "k_implicit_tree<{T}, false>", TREE_GRID: "k_implicit_tree<{T}, true>",
                 TREE_LOCAL: "k_implicit_tree_local<{T}, false>",
-                TREE_LOCAL_LDS: "k_implicit_tree_local<{T}, true>"}
+                TREE_LOCAL_LDS: "k_implicit_tree_local<{T}, true>",
+                TREE_RESIDENT: "k_resident"}
 
 _dp = C.POINTER(C.c_double)
 _ip = C.POINTER(C.c_int32)

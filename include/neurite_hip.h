@@ -222,7 +222,8 @@ typedef struct nrt_stats {
   int32_t num_blocks;       /* persistent kernels: workgroups in the grid       */
   int32_t restarts;         /* Krylov breakdown restarts summed over steps      */
   int32_t tree_form;        /* tree solve launch: NRT_TREE_BLOCK, _GRID, _LOCAL,
-                               _LOCAL_LDS (group-resident), -1 otherwise        */
+                               _LOCAL_LDS (group-resident), _RESIDENT, -1
+                               otherwise                                        */
   int32_t reserved;
 } nrt_stats;
 
@@ -231,6 +232,7 @@ typedef struct nrt_stats {
 #define NRT_TREE_GRID       1  /* level-synchronous grid (a barrier per level)   */
 #define NRT_TREE_LOCAL      2  /* local mode, levels in global memory            */
 #define NRT_TREE_LOCAL_LDS  3  /* local mode, each group's levels in its LDS     */
+#define NRT_TREE_RESIDENT   4  /* rows resident in registers (few rows change)   */
 
 typedef struct nrt_handle nrt_handle;
 
