@@ -671,10 +671,7 @@ int nrt_batch_snapshot(nrt_batch* b, int32_t slot, double* host_out) {
     if (b->is_implicit()) {
       implicit_snapshot(s.h, host_out);
     } else {
-      const double* v = explicit_slot_v(s.h, s.done);
-      NRT_HIP(hipMemcpyAsync(host_out, v, sizeof(double) * s.N, hipMemcpyDeviceToHost,
-                             b->stream));
-      NRT_HIP(hipStreamSynchronize(b->stream));
+      snapshot_to_host(b->device, explicit_slot_v(s.h, s.done), nullptr, s.N, host_out, b->stream);
     }
     return NRT_OK;
   });

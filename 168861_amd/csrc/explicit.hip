@@ -457,9 +457,7 @@ void explicit_step(nrt_handle* hnd, bool active, double* trace_dst, int32_t trac
 
 void explicit_snapshot(nrt_handle* hnd, double* host_out) {
   Explicit* e = hnd->ex;
-  NRT_HIP(hipMemcpyAsync(host_out, e->V[e->cur].p, sizeof(double) * e->N,
-                         hipMemcpyDeviceToHost, hnd->stream));
-  NRT_HIP(hipStreamSynchronize(hnd->stream));
+  snapshot_to_host(hnd->device, e->V[e->cur].p, nullptr, e->N, host_out, hnd->stream);
 }
 
 void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64_t a1,

@@ -101,8 +101,10 @@ struct Implicit {
   DBuf<uint16_t> rinf16;
   DBuf<int32_t> rinf32;
   DBuf<unsigned long long> rll;
+  DBuf<int32_t> rslot_dev;  // rslot on the device (snapshots)
   unsigned rtag = 0;  // tag of the last step launched
   int64_t rsteps = 0;
+  unsigned rerr = 0;  // the last launch gave up
   std::vector<int32_t> rslot;  // element -> index in x
 };
 
@@ -2170,6 +2172,7 @@ static bool resident_create(nrt_handle* hnd, Implicit* e, const HostProblem& p,
   dyn.insert(dyn.end(), P.dyn_s.begin(), P.dyn_s.end());
   dyn.insert(dyn.end(), P.dyn_u.begin(), P.dyn_u.end());
   e->rdyn.upload(dyn, s);
+  e->rslot_dev.upload(P.slot, s);
   e->rll.alloc(4 * (size_t)P.npub);
   NRT_HIP(hipMemsetAsync(e->rll.p, 0, sizeof(unsigned long long) * 4 * P.npub, s));
   r.has_input = inp.empty() ? 0 : 1;
@@ -2898,12 +2901,19 @@ static std::string failure_message(const Implicit* e, const nrt_options& o, cons
 static int collect_stats(nrt_handle* hnd) {
   Implicit* e = hnd->im;
   ImpStats st{};
-  unsigned err = 0;
-  NRT_HIP(hipMemcpyAsync(&st, e->st.p, sizeof(ImpStats), hipMemcpyDeviceToHost, hnd->stream));
-  NRT_HIP(hipMemcpyAsync(&err, e->bar.p + 2, sizeof(unsigned), hipMemcpyDeviceToHost, hnd->stream));
-  NRT_HIP(hipStreamSynchronize(hnd->stream));
-  hnd->stats.steps = e->resident ? e->rsteps : (int64_t)st.steps;
-  hnd->stats.krylov_iters = e->resident ? e->rsteps : (int64_t)st.iters_total;
+  unsigned err = e->rerr;
+  if (!e->resident) {
+    NRT_HIP(hipMemcpyAsync(&st, e->st.p, sizeof(ImpStats), hipMemcpyDeviceToHost, hnd->stream));
+    NRT_HIP(hipMemcpyAsync(&err, e->bar.p + 2, sizeof(unsigned), hipMemcpyDeviceToHost,
+                           hnd->stream));
+    NRT_HIP(hipStreamSynchronize(hnd->stream));
+  } else {  // an exact solve a step: nothing to fetch
+    NRT_HIP(hipStreamSynchronize(hnd->stream));
+    st.steps = st.iters_total = (unsigned long long)e->rsteps;
+    st.last_iters = e->rsteps > 0 ? 1 : 0;
+  }
+  hnd->stats.steps = (int64_t)st.steps;
+  hnd->stats.krylov_iters = (int64_t)st.iters_total;
   hnd->stats.refine_sweeps =
       hnd->opt.precision == NRT_FP32_REFINE || e->method >= 3 ? (int64_t)st.sweeps_total : 0;
   hnd->stats.last_iters = st.last_iters;
@@ -2923,6 +2933,7 @@ static int collect_stats(nrt_handle* hnd) {
     // launch has drained (every workgroup leaves at the flag), so clear them for
     // the handle's next launch.
     reset_barrier(e, hnd->stream);
+    e->rerr = 0;
     throw Error(NRT_ERR_HIP,
                 "grid barrier timed out inside the persistent kernel (its workgroups were not "
                 "all resident at once: another launch held part of the device)");
@@ -2977,6 +2988,7 @@ static void run_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_t 
             100 * std::min(attempt + 1, 50) + (int)((uint32_t)((uintptr_t)e >> 6) * 2654435761u >> 22)));
         continue;
       }
+      e->rerr = err;
       if (err) return;  // collect_stats reports it
     }
     resident_flip(e, num);
@@ -2996,16 +3008,8 @@ int implicit_calculate(nrt_handle* hnd) {
 // one when the caller knows that no queued work writes V).
 void implicit_snapshot_on(nrt_handle* hnd, double* host_out, hipStream_t s) {
   Implicit* e = hnd->im;
-  if (e->method == 0) {
-    NRT_HIP(hipMemcpyAsync(host_out, e->x.p, sizeof(double) * e->N, hipMemcpyDeviceToHost, s));
-    NRT_HIP(hipStreamSynchronize(s));
-    return;
-  }
-  std::vector<double> xs(e->ns0);  // slot order -> element order
-  NRT_HIP(hipMemcpyAsync(xs.data(), e->x.p, sizeof(double) * e->ns0, hipMemcpyDeviceToHost, s));
-  NRT_HIP(hipStreamSynchronize(s));
-  const int32_t* s0 = e->resident ? e->rslot.data() : e->plan_h.slot0.data();
-  for (int i = 0; i < e->N; i++) host_out[i] = xs[s0[i]];
+  const int32_t* slot = e->method == 0 ? nullptr : e->resident ? e->rslot_dev.p : e->plan.slot0;
+  snapshot_to_host(hnd->device, e->x.p, slot, e->N, host_out, s);
 }
 
 void implicit_snapshot(nrt_handle* hnd, double* host_out) {

@@ -138,6 +138,10 @@ int implicit_run(nrt_handle* h, int64_t first, int64_t num, int64_t a0, int64_t 
 
 inline int grid_for(int64_t n, int block) { return (int)((n + block - 1) / block); }
 
+// snapshot.hip
+void snapshot_to_host(int device, const double* x, const int32_t* slot, int n, double* out,
+                      hipStream_t s);
+
 // capi.cpp
 int pick_device(int requested);
 nrt_options resolve_options(const nrt_options* opt);  // defaults + validation
