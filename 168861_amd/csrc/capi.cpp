@@ -145,7 +145,7 @@ nrt_handle* handle_create(const nrt_problem* p, const nrt_options& o, hipStream_
     } else {
       NRT_HIP(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
     }
-    if (o.kind == NRT_EXPLICIT) h->ex = explicit_create(h, q);
+    if (o.kind == NRT_EXPLICIT) h->ex = explicit_create(h, q, shared != nullptr);
     else h->im = implicit_create(h, q, batch_threads);
   } catch (...) {
     if (h->stream && h->owns_stream) (void)hipStreamDestroy(h->stream);

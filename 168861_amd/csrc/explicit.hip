@@ -24,43 +24,9 @@
 // is exp() (device libm vs host libm, both within an ulp or so).
 #include <algorithm>
 #include <cstring>
-#include "nrt_internal.hpp"
+#include "explicit_dev.hpp"
 
 namespace nrt {
-
-struct HHDev {
-  double* m;
-  double* h;
-  double* n;
-  const double* E_Na;
-  const double* E_K;
-  const double* E_L;
-  const double* g_Na;
-  const double* g_K;
-  const double* G_L;
-  const double* ls_Na;
-  const double* ls_K;
-  const double* rest;
-  const double* dx;
-};
-
-struct Explicit {
-  int N = 0, H = 0, R = 0;
-  double dT = 0, dt_ms = 0;
-  DBuf<double> V[2];
-  DBuf<double> coefA, rdx, wdx, kdx;
-  DBuf<uint32_t> code;
-  DBuf<ExRec> recs;
-  DBuf<double> m, h, n, E_Na, E_K, E_L, g_Na, g_K, G_L, ls_Na, ls_K, rest, hdx;
-  DBuf<double> trace;
-  int cur = 0;  // buffer holding the latest potential (the reference's prevT)
-  int64_t trace_cap = 0;
-  bool res_attr = false;  // the resident kernel's LDS limit is raised
-  HHDev hd() {
-    return HHDev{m.p, h.p, n.p, E_Na.p, E_K.p, E_L.p, g_Na.p, g_K.p, G_L.p, ls_Na.p, ls_K.p,
-                 rest.p, hdx.p};
-  }
-};
 
 // Forward-Euler HH gating of HH element i at potential v (solverEx-cpu.cpp:62-82,
 // coupling.cpp:25-48, discretization.cpp:81-86); returns W*dx and K*dx.
@@ -110,15 +76,6 @@ template <class X>
 __device__ __forceinline__ void ready_s(X x) {
   asm volatile("" ::"s"(x));
 }
-
-// Element kinds of the explicit step (code >> 29; the low 29 bits are an index):
-// the flag bits kCodeHH, kCodeRec, kCodeSkip alone or HH with Skip keep their
-// meaning (chain element, HH chain element with its HH index, exception record,
-// terminal/ghost); the three unused combinations carry an element with one
-// exception and no record: a daughter (index = its mother), a branch point (index =
-// its left daughter), a source of the sealed end right after it (no index).
-constexpr uint32_t kExPlain = 0, kExSkip = 1, kExRecord = 2, kExBranch = 3, kExHH = 4,
-                   kExSkipHH = 5, kExDaughter = 6, kExCopyNext = 7;
 
 // Explicit step of element j of N: reads Vo, writes Vn[j] and its sealed-end copies.
 // A plain chain element (no record) couples to j - 1 and j + 1; its operands are
@@ -274,7 +231,6 @@ __global__ __launch_bounds__(256) void k_explicit_fp64(
 // kernel launches (a launch per step costs more than a thousand elements' work).
 // The element update is explicit_element's, operand for operand.
 constexpr int kResBlock = 1024;
-constexpr int kResMaxN = 8192;  // two potentials of 8 B: 128 KiB of LDS
 
 __global__ __launch_bounds__(kResBlock) void k_explicit_resident(
     int N, const double* __restrict__ Vin, const double* __restrict__ Vother,
@@ -314,7 +270,7 @@ __global__ __launch_bounds__(kResBlock) void k_explicit_resident(
   for (int j = tid; j < N; j += nt) Vout[j] = A[j];
 }
 
-Explicit* explicit_create(nrt_handle* hnd, const HostProblem& p) {
+Explicit* explicit_create(nrt_handle* hnd, const HostProblem& p, bool in_batch) {
   hipStream_t s = hnd->stream;
   const int N = p.N, H = p.H;
   auto* e = new Explicit;
@@ -426,6 +382,7 @@ Explicit* explicit_create(nrt_handle* hnd, const HostProblem& p) {
     e->ls_K.upload(p.ls_K, s);
     e->rest.upload(p.rest, s);
     e->hdx.upload(hdx, s);
+    cable_prepare(hnd, e, p, in_batch);
     NRT_HIP(hipStreamSynchronize(s));
   } catch (...) {
     delete e;
@@ -474,7 +431,13 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
   NRT_HIP(hipEventCreate(&t1));
   NRT_HIP(hipEventRecord(t0, hnd->stream));
   int64_t k = 0;
-  if (e->N <= kResMaxN) {
+  int64_t launches = num;
+  if (cable_run(hnd, e, first, num, a0, a1, tracing ? trace_elem : 0, interval,
+                tracing && trace_out ? e->trace.p : nullptr, t0, t1)) {
+    k = max_samples;
+    launches = 1;
+  } else if (e->N <= kResMaxN) {
+    launches = 1;
     // one launch for the whole run; the result lands in the other buffer, which
     // becomes the current one (the flips of num steps, then one more)
     const size_t lds = sizeof(double) * 2 * (size_t)e->N;
@@ -506,7 +469,7 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
       explicit_step(hnd, active, dst, trace_elem);
     }
   }
-  NRT_HIP(hipEventRecord(t1, hnd->stream));
+  if (e->cable_groups == 0) NRT_HIP(hipEventRecord(t1, hnd->stream));
   if (trace_out && k > 0)
     NRT_HIP(hipMemcpyAsync(trace_out, e->trace.p, sizeof(double) * k, hipMemcpyDeviceToHost,
                            hnd->stream));
@@ -516,7 +479,7 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
   hnd->stats.kernel_ms = ms;
-  hnd->stats.kernel_launches = e->N <= kResMaxN ? 1 : num;
+  hnd->stats.kernel_launches = launches;
   hnd->stats.steps += num;
   if (ns) *ns = k;
 }

@@ -120,7 +120,8 @@ struct nrt_handle {
 
 namespace nrt {
 // explicit.hip
-Explicit* explicit_create(nrt_handle* h, const HostProblem& p);
+// in_batch: a slot of a batch (stepped by the batch's launches only).
+Explicit* explicit_create(nrt_handle* h, const HostProblem& p, bool in_batch = false);
 void explicit_destroy(Explicit* e);
 void explicit_step(nrt_handle* h, bool active, double* trace_dst, int32_t trace_elem);
 void explicit_snapshot(nrt_handle* h, double* host_out);
