@@ -50,6 +50,17 @@ void explicit_batch_steps(const void* slots, const int2* blk, int nblk, int nslo
 const double* explicit_slot_v(nrt_handle* h, long long done);
 int64_t explicit_device_bytes(const Explicit* e);
 int explicit_batch_block_elems();
+// explicit_tree.hip
+bool explicit_tree_slot(const nrt_handle* h);
+size_t explicit_tree_rec_bytes();
+size_t explicit_tree_work_bytes();
+void explicit_tree_shape(nrt_handle* h, int* groups, int* T);
+void explicit_tree_fill(nrt_handle* h, unsigned* err, long long a0, long long a1, int trace_elem,
+                        long long interval, double* trace, void* out);
+void explicit_tree_work(nrt_handle* h, long long done, long long steps, void* out);
+void explicit_tree_undo(nrt_handle* h, const void* work, long long* steps);
+void explicit_tree_batch_launch(const void* recs, const void* work, const int2* map,
+                                unsigned* ticket, int nwg, int T, hipStream_t s);
 
 namespace {
 // Workgroup sizes the autotuner tries, in this order, for each size class of slots.
@@ -75,6 +86,7 @@ constexpr int64_t kAdmissionReserve = 512ll << 20;  // left free for the runtime
 // in a launch of their own while they fill the device: a workgroup of the large ones'
 // size would leave two thirds of its waves idle.
 constexpr int kResSmallT = 192;
+constexpr int kExSmallFill = 1024;  // explicit slots of that size that fill the device
 struct ResStep {  // ResWork of resident_dev.hpp
   long long done, steps;
 };
@@ -116,9 +128,9 @@ struct nrt_batch {
   long long g = 0;                           // batch steps done
   bool dirty = true;
   std::vector<int> order;  // slot ids in table order
-  // implicit: the slots whose tree solve is resident, by unit threads per workgroup
-  // (small ones apart), largest first; per launch their steps, the workgroups' (slot,
-  // group) map and a ticket, in one upload
+  // the slots whose rows stay in registers (implicit: the resident tree solve; explicit:
+  // trees), by unit threads per workgroup (small ones apart), largest first, and the
+  // workgroups' (slot, group) map; per launch their steps and a ticket, in one upload
   struct ResClass {
     std::vector<int> ids;
     int T = 0, maxG = 0;  // most unit threads, most workgroups of a slot
@@ -127,7 +139,9 @@ struct nrt_batch {
   };
   ResClass res[2];
   DBuf<uint8_t> rtable, rwork;
+  DBuf<int2> rmap;
   std::vector<uint8_t> rwork_h;
+  HostWord rerr;  // explicit: an exchange timed out
   DBuf<uint8_t> table;
   DBuf<int2> blk;
   int nblk = 0;
@@ -218,6 +232,7 @@ struct nrt_batch {
       work_h.resize(order.size() * implicit_slot_work_bytes());
       vn.assign(order.size(), 1);
     } else {
+      rebuild_resident();
       const size_t sb = explicit_slot_bytes();
       std::vector<uint8_t> host(sb * order.size());
       std::vector<int2> bl;
@@ -243,13 +258,13 @@ struct nrt_batch {
     for (ResClass& c : res) c = ResClass();
     std::vector<int> rest;
     for (int id : order) {
-      if (!implicit_resident(slots[id]->h)) {
+      if (!row_resident(id)) {
         rest.push_back(id);
         continue;
       }
       int G = 0, T = 0;
       size_t lds = 0;
-      resident_slot_shape(slots[id]->h, &G, &T, &lds);
+      shape(id, G, T, lds);
       ResClass& c = res[T <= kResSmallT ? 1 : 0];
       c.ids.push_back(id);
       c.T = std::max(c.T, T);
@@ -258,26 +273,52 @@ struct nrt_batch {
     }
     order.swap(rest);
     if (!res[0].ids.empty() && !res[1].ids.empty() &&
-        (int)res[1].ids.size() < resident_capacity(device, res[1].T, res[1].lds) / 2) {
+        (int)res[1].ids.size() <
+            (is_implicit() ? resident_capacity(device, res[1].T, res[1].lds) : kExSmallFill) / 2) {
       res[0].ids.insert(res[0].ids.end(), res[1].ids.begin(), res[1].ids.end());
       res[0].lds = std::max(res[0].lds, res[1].lds);
       res[0].maxG = std::max(res[0].maxG, res[1].maxG);
       res[1] = ResClass();
     }
-    const size_t rb = resident_rec_bytes();
+    const size_t rb = is_implicit() ? resident_rec_bytes() : explicit_tree_rec_bytes();
+    if (!is_implicit()) rerr.take();
     std::vector<uint8_t> host;
+    std::vector<int2> map;
+    int at = 0;
     for (ResClass& c : res) {
       std::stable_sort(c.ids.begin(), c.ids.end(),
                        [&](int a, int b) { return slots[a]->N > slots[b]->N; });
+      c.map_at = map.size();
       for (int id : c.ids) {
         Slot& s = *slots[id];
+        int G = 0, T = 0;
+        size_t lds = 0;
+        shape(id, G, T, lds);
+        for (int g = 0; g < G; g++) map.push_back(make_int2(at, g));
+        at++;
         host.resize(host.size() + rb);
-        resident_slot_fill(s.h, s.a0, s.a1, s.trace_elem, s.interval, s.trace.p,
-                           host.data() + host.size() - rb);
+        uint8_t* out = host.data() + host.size() - rb;
+        if (is_implicit())
+          resident_slot_fill(s.h, s.a0, s.a1, s.trace_elem, s.interval, s.trace.p, out);
+        else
+          explicit_tree_fill(s.h, rerr.p, s.a0, s.a1, s.trace_elem, s.interval, s.trace.p, out);
       }
+      c.nwg = (int)(map.size() - c.map_at);
     }
     rtable.upload(host, stream);
+    rmap.upload(map, stream);
     NRT_HIP(hipStreamSynchronize(stream));
+  }
+
+  bool row_resident(int id) const {
+    return is_implicit() ? implicit_resident(slots[id]->h) : explicit_tree_slot(slots[id]->h);
+  }
+  void shape(int id, int& G, int& T, size_t& lds) const {
+    if (is_implicit()) resident_slot_shape(slots[id]->h, &G, &T, &lds);
+    else explicit_tree_shape(slots[id]->h, &G, &T);
+  }
+  size_t work_bytes() const {
+    return is_implicit() ? sizeof(ResStep) : explicit_tree_work_bytes();
   }
 
   // Enqueues the resident slots' steps (largest workgroups first).
@@ -285,41 +326,40 @@ struct nrt_batch {
                        int64_t& ss) {
     const size_t n = res[0].ids.size() + res[1].ids.size();
     if (n == 0) return;
-    std::vector<int2> map;
-    rwork_h.assign(n * sizeof(ResStep), 0);
+    const size_t wb = work_bytes();
+    rwork_h.assign(n * wb + 4 * sizeof(unsigned), 0);  // steps, tickets
+    const size_t tick_at = n * wb;
     size_t at = 0;
-    for (ResClass& c : res) {
-      c.map_at = map.size();
+    for (ResClass& c : res)
       for (int id : c.ids) {
         Slot& s = *slots[id];
-        int G = 0, T = 0;
-        size_t lds = 0;
-        resident_slot_shape(s.h, &G, &T, &lds);
         long long want = k;
-        if (elem_budget > 0)
+        if (elem_budget > 0) {
+          int G = 0, T = 0;
+          size_t lds = 0;
+          shape(id, G, T, lds);
           want = std::max(1ll, std::min(kmax > 0 ? kmax : k, elem_budget * G / std::max(1, s.N)));
+        }
+        // (at least one step: the table holds slots with steps left only)
         const ResStep w{s.done, std::min(want, s.left())};
-        memcpy(rwork_h.data() + at * sizeof(ResStep), &w, sizeof(w));
-        if (w.steps > 0)
-          for (int g = 0; g < G; g++) map.push_back(make_int2((int)at, g));
+        if (is_implicit()) memcpy(rwork_h.data() + at * wb, &w, sizeof(w));
+        else explicit_tree_work(s.h, w.done, w.steps, rwork_h.data() + at * wb);
         s.done += w.steps;
         ss += w.steps;
         cs += w.steps * s.N;
         at++;
       }
-      c.nwg = (int)(map.size() - c.map_at);
-    }
-    // steps, map, tickets
-    const size_t map_at = rwork_h.size(), tick_at = map_at + map.size() * sizeof(int2);
-    rwork_h.resize(tick_at + 2 * sizeof(int2), 0);
-    memcpy(rwork_h.data() + map_at, map.data(), map.size() * sizeof(int2));
     if (rwork.n < rwork_h.size()) rwork.alloc(2 * rwork_h.size());
     NRT_HIP(hipMemcpyAsync(rwork.p, rwork_h.data(), rwork_h.size(), hipMemcpyHostToDevice, stream));
     for (int c = 0; c < 2; c++) {
       if (res[c].nwg == 0) continue;
-      resident_batch_launch(rtable.p, rwork.p, (const int2*)(rwork.p + map_at) + res[c].map_at,
-                            (unsigned*)(rwork.p + tick_at) + 2 * c, res[c].nwg, res[c].T,
-                            res[c].lds, stream);
+      const int2* m = rmap.p + res[c].map_at;
+      unsigned* ticket = (unsigned*)(rwork.p + tick_at) + 2 * c;
+      if (is_implicit())
+        resident_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, res[c].lds,
+                              stream);
+      else
+        explicit_tree_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, stream);
       pend_launches++;
     }
   }
@@ -350,7 +390,7 @@ struct nrt_batch {
       // (the ticket leaves at most one neurite's workgroups waiting for others to start)
       int most = 0;
       for (const ResClass& c : res) most = std::max(most, c.maxG);
-      held = device_share(device, order.empty() ? most : INT_MAX);
+      held = device_share(device, order.empty() || !is_implicit() ? most : INT_MAX);
       NRT_HIP(hipEventRecord(ev0, stream));
       launch_resident(k, elem_budget, kmax, cs, ss);
       if (order.empty()) {
@@ -470,10 +510,10 @@ struct nrt_batch {
       // launches take it from device memory, set here before each replay
       gbase_h = g - k;
       NRT_HIP(hipMemcpyAsync(gdev.p, &gbase_h, sizeof(long long), hipMemcpyHostToDevice, stream));
-      NRT_HIP(hipEventRecord(ev0, stream));
+      if (!any_resident()) NRT_HIP(hipEventRecord(ev0, stream));
       NRT_HIP(hipGraphLaunch(gexec, stream));
       NRT_HIP(hipEventRecord(ev1, stream));
-      pend_launches = k;
+      pend_launches += k;
     }
     pend_cs = cs;
     pend_ss = ss;
@@ -529,6 +569,23 @@ struct nrt_batch {
     return seg;
   }
 
+  // Explicit slots of several workgroups: if an exchange timed out, every resident slot is
+  // where it was before the launch, and an error says so.
+  void check_exchanges() {
+    if (!rerr.p || !rerr.get()) return;
+    rerr.clear();
+    size_t at = 0;
+    for (ResClass& c : res)
+      for (int id : c.ids) {
+        long long steps = 0;
+        explicit_tree_undo(slots[id]->h, rwork_h.data() + at++ * work_bytes(), &steps);
+        slots[id]->done -= steps;
+      }
+    throw Error(NRT_ERR_HIP,
+                "exchange timed out inside an explicit batch kernel (another launch held part "
+                "of the device); the slots are where they were before this launch");
+  }
+
   // Waits for the launch in flight and accounts for it.
   void finish() {
     if (!pending) return;
@@ -558,6 +615,7 @@ struct nrt_batch {
     } else {
       NRT_HIP(hipEventSynchronize(ev1));
       NRT_HIP(hipEventElapsedTime(&ms, ev0, ev1));
+      check_exchanges();
     }
     stats.launches += pend_launches;
     stats.kernel_ms += ms;

@@ -383,6 +383,7 @@ Explicit* explicit_create(nrt_handle* hnd, const HostProblem& p, bool in_batch) 
     e->rest.upload(p.rest, s);
     e->hdx.upload(hdx, s);
     cable_prepare(hnd, e, p, in_batch);
+    if (e->cable_groups == 0) tree_prepare(hnd, e, p, in_batch);
     NRT_HIP(hipStreamSynchronize(s));
   } catch (...) {
     delete e;
@@ -432,8 +433,11 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
   NRT_HIP(hipEventRecord(t0, hnd->stream));
   int64_t k = 0;
   int64_t launches = num;
-  if (cable_run(hnd, e, first, num, a0, a1, tracing ? trace_elem : 0, interval,
-                tracing && trace_out ? e->trace.p : nullptr, t0, t1)) {
+  double* const trace = tracing && trace_out ? e->trace.p : nullptr;
+  const int32_t probe = tracing ? trace_elem : 0;
+  const bool exchanging = cable_run(hnd, e, first, num, a0, a1, probe, interval, trace, t0, t1) ||
+                          tree_run(hnd, e, first, num, a0, a1, probe, interval, trace, t0, t1);
+  if (exchanging) {
     k = max_samples;
     launches = 1;
   } else if (e->N <= kResMaxN) {
@@ -451,8 +455,7 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
                        e->V[e->cur].p, e->V[1 - e->cur].p, e->V[1 - e->cur].p, e->coefA.p,
                        e->rdx.p, e->wdx.p, e->kdx.p, e->code.p, e->recs.p, e->hd(), e->dt_ms,
                        (long long)first, (long long)num, (long long)a0, (long long)a1,
-                       tracing ? trace_elem : 0, (long long)interval,
-                       tracing && trace_out ? e->trace.p : nullptr);
+                       probe, (long long)interval, trace);
     NRT_HIP(hipGetLastError());
     e->cur = 1 - e->cur;
     k = max_samples;
@@ -469,7 +472,7 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
       explicit_step(hnd, active, dst, trace_elem);
     }
   }
-  if (e->cable_groups == 0) NRT_HIP(hipEventRecord(t1, hnd->stream));
+  if (!exchanging) NRT_HIP(hipEventRecord(t1, hnd->stream));
   if (trace_out && k > 0)
     NRT_HIP(hipMemcpyAsync(trace_out, e->trace.p, sizeof(double) * k, hipMemcpyDeviceToHost,
                            hnd->stream));
@@ -630,6 +633,7 @@ void explicit_batch_steps(const void* slots, const int2* blk, int nblk, int nslo
 // Buffer holding V of a slot after `done` of its steps.
 const double* explicit_slot_v(nrt_handle* h, long long done) {
   Explicit* e = h->ex;
+  if (e->tree_groups > 0) return e->V[e->cur].p;  // (its launches flip the buffers)
   return e->V[(e->cur + (int)(done & 1)) & 1].p;
 }
 

@@ -30,13 +30,6 @@ constexpr int kCabHalo = 8;
 constexpr int kCabOwn = kCabBlock - 2 * kCabHalo;
 constexpr int kCabState = 4;  // V, m, h, n
 
-// x / c from y = 1 / c (rounded): the quotient's first estimate, its exact remainder,
-// one correction.
-__device__ __forceinline__ double div_by(double x, double c, double y) {
-  const double q = x * y;
-  return fma(fma(-c, q, x), y, q);
-}
-
 struct CabArgs {
   int N, G;
   const double* Vin;
@@ -55,15 +48,6 @@ struct CabArgs {
   unsigned tag0;
   unsigned long long first_limit, limit;
 };
-
-// Both words of a value carry the exchange's tag (see resident.hip).
-__device__ __forceinline__ void cab_put(unsigned long long* w, unsigned tag, double v) {
-  const unsigned long long t = (unsigned long long)tag << 32;
-  __hip_atomic_store(w, t | (unsigned)__double2loint(v), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(w + 1, t | (unsigned)__double2hiint(v), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
 
 __global__ __launch_bounds__(kCabBlock) void k_explicit_cable(CabArgs q) {
   __shared__ double sv[2][kCabBlock + 2];  // one more on either side: never valid
@@ -139,57 +123,40 @@ __global__ __launch_bounds__(kCabBlock) void k_explicit_cable(CabArgs q) {
     if (halo && left == 0) {
       left = halo;
       tag++;
-      unsigned long long* ll =
-          q.ll + (size_t)(tag & 1) * q.G * 2 * kCabHalo * kCabState * 2;
+      ExWord* ll =
+          (ExWord*)q.ll + (size_t)(tag & 1) * q.G * 2 * kCabHalo * kCabState * 2;
       auto at = [&](int gg, int side, int kk) {
         return ll + ((((size_t)gg * 2 + side) * kCabHalo + kk) * kCabState) * 2;
       };
       if (put_l) {
-        unsigned long long* o = at(g, 0, t - halo);
-        cab_put(o, tag, v);
+        ExWord* o = at(g, 0, t - halo);
+        ex_put(o, tag, v);
         if (hh >= 0) {
-          cab_put(o + 2, tag, m);
-          cab_put(o + 4, tag, h);
-          cab_put(o + 6, tag, n);
+          ex_put(o + 2, tag, m);
+          ex_put(o + 4, tag, h);
+          ex_put(o + 6, tag, n);
         }
       }
       if (put_r) {
-        unsigned long long* o = at(g, 1, t - (kCabBlock - 2 * halo));
-        cab_put(o, tag, v);
+        ExWord* o = at(g, 1, t - (kCabBlock - 2 * halo));
+        ex_put(o, tag, v);
         if (hh >= 0) {
-          cab_put(o + 2, tag, m);
-          cab_put(o + 4, tag, h);
-          cab_put(o + 6, tag, n);
+          ex_put(o + 2, tag, m);
+          ex_put(o + 4, tag, h);
+          ex_put(o + 6, tag, n);
         }
       }
+      __builtin_amdgcn_wave_barrier();  // a wave's lanes all put before any waits
       if (get) {
-        const unsigned long long* o = at(src_g, src_side, src_k);
-        const int nw = hh >= 0 ? 2 * kCabState : 2;
-        const unsigned long long most = first_ex ? q.first_limit : q.limit;
-        unsigned long long x[2 * kCabState], spins = 0;
-        while (true) {
-          bool all = true;
-#pragma unroll
-          for (int e = 0; e < 2 * kCabState; e++)
-            if (e < nw) {
-              x[e] = __hip_atomic_load(o + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              all = all && (unsigned)(x[e] >> 32) == tag;
-            }
-          if (all) break;
-          // bounded; once another workgroup gave up, all do
-          if (++spins > most ||
-              ((spins & 255) == 0 &&
-               __hip_atomic_load(q.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
-            __hip_atomic_store(q.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            fail = 1;
-            break;
-          }
-        }
-        v = __hiloint2double((int)(unsigned)x[1], (int)(unsigned)x[0]);
+        const ExWord* o = at(src_g, src_side, src_k);
+        double x[kCabState] = {};
+        if (!ex_get(o, tag, hh >= 0 ? kCabState : 1, first_ex ? q.first_limit : q.limit, q.err, x))
+          fail = 1;
+        v = x[0];
         if (hh >= 0) {
-          m = __hiloint2double((int)(unsigned)x[3], (int)(unsigned)x[2]);
-          h = __hiloint2double((int)(unsigned)x[5], (int)(unsigned)x[4]);
-          n = __hiloint2double((int)(unsigned)x[7], (int)(unsigned)x[6]);
+          m = x[1];
+          h = x[2];
+          n = x[3];
         }
       }
       first_ex = false;
@@ -284,54 +251,66 @@ void cable_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_b
   e->m2.alloc(p.H);
   e->h2.alloc(p.H);
   e->n2.alloc(p.H);
-  e->err.alloc(1);
-  NRT_HIP(hipMemsetAsync(e->err.p, 0, sizeof(unsigned), hnd->stream));
+  e->err.take();
   if (G > 1) {
     e->ll.alloc((size_t)2 * G * 2 * kCabHalo * kCabState * 2);
     NRT_HIP(hipMemsetAsync(e->ll.p, 0, sizeof(unsigned long long) * e->ll.n, hnd->stream));
   }
 }
 
-bool cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
-               int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
-               hipEvent_t t1) {
-  if (e->cable_groups == 0) return false;
-  const int G = e->cable_groups;
+void run_exchanging(nrt_handle* hnd, Explicit* e, int G,
+                    const std::function<void(unsigned long long, unsigned long long)>& launch,
+                    hipEvent_t t0, hipEvent_t t1) {
   unsigned long long limit = 1ull << 28;
   const char* sl = getenv("NRT_SPIN_LIMIT");
   if (sl) limit = strtoull(sl, nullptr, 10);
   const auto share = device_share(hnd->device, G > 1 ? G : 0);
   const auto until = std::chrono::steady_clock::now() + std::chrono::seconds(sl ? 1 : 180);
   for (int attempt = 0;; attempt++) {
-    CabArgs q{e->N, G, e->V[e->cur].p, e->V[1 - e->cur].p, e->coefA.p, e->rdx.p, e->wdx.p,
-              e->kdx.p, e->code.p, e->recs.p, e->hd(), e->m2.p, e->h2.p, e->n2.p, e->dt_ms,
-              (long long)first, (long long)num, (long long)a0, (long long)a1,
-              (long long)interval, trace_elem, trace, e->ll.p, e->err.p, e->tag,
-              std::min(limit, 20000ull), limit};
-    e->tag += (unsigned)(num / kCabHalo + 2);
     NRT_HIP(hipEventRecord(t0, hnd->stream));
-    hipLaunchKernelGGL(k_explicit_cable, dim3(G), dim3(kCabBlock), 0, hnd->stream, q);
+    launch(std::min(limit, 20000ull), limit);
     NRT_HIP(hipGetLastError());
     NRT_HIP(hipEventRecord(t1, hnd->stream));
-    unsigned err = 0;
-    if (G > 1) {
-      NRT_HIP(hipMemcpyAsync(&err, e->err.p, sizeof(unsigned), hipMemcpyDeviceToHost, hnd->stream));
-      NRT_HIP(hipStreamSynchronize(hnd->stream));
-    }
-    if (!err) break;
+    if (G == 1) break;
+    NRT_HIP(hipStreamSynchronize(hnd->stream));
+    if (!e->err.get()) break;
     // workgroups that did not all start in time (another process holds part of the
-    // device): nothing was stored, the run is tried again
-    NRT_HIP(hipMemsetAsync(e->err.p, 0, sizeof(unsigned), hnd->stream));
+    // device): nothing that counts was stored, the run is tried again
+    e->err.clear();
     NRT_REQUIRE(std::chrono::steady_clock::now() < until, NRT_ERR_HIP,
-                "exchange timed out inside the cable kernel (its workgroups were not all "
+                "exchange timed out inside an explicit kernel (its workgroups were not all "
                 "resident at once: another launch held part of the device)");
     std::this_thread::sleep_for(std::chrono::microseconds(
         100 * std::min(attempt + 1, 50) + (int)((uint32_t)((uintptr_t)e >> 6) * 2654435761u >> 22)));
   }
+  // the run's results become the current ones
   e->cur = 1 - e->cur;
   std::swap(e->m.p, e->m2.p);
   std::swap(e->h.p, e->h2.p);
   std::swap(e->n.p, e->n2.p);
+}
+
+bool cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
+               int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
+               hipEvent_t t1) {
+  // One step of a short neurite, or two of a very short one, are done by one workgroup
+  // before this launch has set up its registers (runs of 1 / 2 / 4 steps there and here, us,
+  // with the launch and the wait: 402 elements 19 / 22 / 30 and 24 / 24 / 26, 1,002
+  // 21 / 26 / 36 and 24 / 25 / 27, 5,000 35 / 53 / 89 and 25 / 25 / 27).
+  if (e->cable_groups == 0 || (num <= 2 && num * e->N <= 2048)) return false;
+  const int G = e->cable_groups;
+  run_exchanging(
+      hnd, e, G,
+      [&](unsigned long long first_limit, unsigned long long limit) {
+        CabArgs q{e->N, G, e->V[e->cur].p, e->V[1 - e->cur].p, e->coefA.p, e->rdx.p, e->wdx.p,
+                  e->kdx.p, e->code.p, e->recs.p, e->hd(), e->m2.p, e->h2.p, e->n2.p, e->dt_ms,
+                  (long long)first, (long long)num, (long long)a0, (long long)a1,
+                  (long long)interval, trace_elem, trace, e->ll.p, e->err.p, e->tag,
+                  first_limit, limit};
+        e->tag += (unsigned)(num / kCabHalo + 2);
+        hipLaunchKernelGGL(k_explicit_cable, dim3(G), dim3(kCabBlock), 0, hnd->stream, q);
+      },
+      t0, t1);
   return true;
 }
 

@@ -68,6 +68,19 @@ struct DBuf {
   void upload(const std::vector<T>& v, hipStream_t s) { upload(v.data(), v.size(), s); }
 };
 
+// A word of pinned host memory that kernels on any device can write (pool.cpp): a launch's
+// complaint that the host reads without a copy. Zero when handed out.
+struct HostWord {
+  unsigned* p = nullptr;
+  HostWord() = default;
+  HostWord(const HostWord&) = delete;
+  HostWord& operator=(const HostWord&) = delete;
+  ~HostWord();
+  void take();
+  unsigned get() const { return *(const volatile unsigned*)p; }
+  void clear() { *(volatile unsigned*)p = 0u; }
+};
+
 // Topology exception record of the explicit step: every element whose
 // neighbourhood is not the plain chain (mother j-1, right daughter j+1, no left
 // daughter, no stimulus, no sealed-end copy) carries one.

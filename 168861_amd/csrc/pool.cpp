@@ -106,4 +106,38 @@ int64_t pool_trim(int device) {
   return n;
 }
 
+// Pages of pinned words, kept for the process; a page is added when every word is in use.
+namespace {
+struct Words {
+  std::mutex mu;
+  std::vector<unsigned*> idle;
+};
+Words& words() {
+  static Words* w = new Words;  // never destroyed: used until the process ends
+  return *w;
+}
+}  // namespace
+
+void HostWord::take() {
+  if (p) return;
+  Words& w = words();
+  std::lock_guard<std::mutex> g(w.mu);
+  if (w.idle.empty()) {
+    unsigned* page = nullptr;
+    const int n = 4096 / 64;  // a cache line each
+    NRT_HIP(hipHostMalloc((void**)&page, 4096, hipHostMallocPortable));
+    for (int i = 0; i < n; i++) w.idle.push_back(page + 16 * i);
+  }
+  p = w.idle.back();
+  w.idle.pop_back();
+  clear();
+}
+
+HostWord::~HostWord() {
+  if (!p) return;
+  Words& w = words();
+  std::lock_guard<std::mutex> g(w.mu);
+  w.idle.push_back(p);
+}
+
 }  // namespace nrt
