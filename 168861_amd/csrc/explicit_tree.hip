@@ -426,7 +426,8 @@ void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_ba
   bool fits = false;
   const int cap = tree_capacity(hnd->device, kExT);
   const auto plan = [&](int T, int most) {
-    if (p.N / kExC > (int64_t)most * T) return;
+    // (strands of some 50 elements and halos: 4 to 6% more units than N / kExC)
+    if (p.N / kExC * 1.03 > (double)most * T) return;
     if (build_explicit_plan(p, T, P, why)) fits = P.G <= most;
   };
   plan(kExTBatch, cap);

@@ -36,6 +36,7 @@
 #include <type_traits>
 #include "nrt_internal.hpp"
 #include "nrt_device.hpp"
+#include "chain.hpp"
 #include "resident_dev.hpp"
 #include "tree.hpp"
 
@@ -105,7 +106,10 @@ struct Implicit {
   unsigned rtag = 0;  // tag of the last step launched
   int64_t rsteps = 0;
   unsigned rerr = 0;  // the last launch gave up
-  std::vector<int32_t> rslot;  // element -> index in x
+  std::vector<int32_t> rslot;  // element -> index in x (empty: the element itself)
+  // unbranched neurites (chain.hip; resident is set too)
+  bool chain = false;
+  ChainDev cdev{};
 };
 
 // ------------------------------------------------------------------ assembly
@@ -2211,6 +2215,91 @@ static bool resident_create(nrt_handle* hnd, Implicit* e, const HostProblem& p,
   return true;
 }
 
+// The chain form (chain.hip) of a FP64 direct solve: unbranched neurites with more gating
+// rows than the resident form takes, up to 64 waves of 512 (or 1,024) rows. Per step,
+// 1,012 rows with 10 nodes 43.7 us in block form, 3.8 here; 10,102 rows with 100 nodes
+// 69 and 5.4; 20,202 rows with 200 nodes 32.6 (local form) and 5.9; 60,602 rows with 600
+// nodes 46.7 and 6.8.
+static bool chain_create(nrt_handle* hnd, Implicit* e, const HostProblem& p,
+                         const std::vector<int32_t>& par, const std::vector<int32_t>& rowptr,
+                         const std::vector<int32_t>& col, const std::vector<double>& cmdx,
+                         const std::vector<double>& kdx) {
+  const nrt_options& o = hnd->opt;
+  const int N = e->N, H = e->H;
+  hipStream_t s = hnd->stream;
+  const int C = N <= kChWaves * 64 * 8 ? 8 : 16, W = grid_for(N, 64 * C);
+  if (o.num_blocks != 0 || o.chunk != 0 || o.chunk_hi != 0 || o.tree_groups != 0 ||
+      o.batch_threads != 0 || H == 0 || W > kChWaves)
+    return false;
+  for (int i = 1; i < N; i++)
+    if (par[i] >= 0 && par[i] != i - 1) return false;  // (the ends are rows of their own)
+  std::vector<int32_t> woff(W + 1, 0);
+  std::vector<std::pair<int32_t, int32_t>> rows;
+  for (int k = 0; k < H; k++) {
+    rows.push_back({p.hh_elem[k], k});
+    woff[p.hh_elem[k] / (64 * C) + 1]++;
+  }
+  std::sort(rows.begin(), rows.end());
+  for (int w = 0; w < W; w++) {
+    if (woff[w + 1] > kChGates) return false;
+    woff[w + 1] += woff[w];
+  }
+  int cus = 0;
+  NRT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, hnd->device));
+  if (W > cus) return false;
+  std::vector<double> val(e->nnz);
+  std::vector<int32_t> type(H);
+  NRT_HIP(hipMemcpyAsync(val.data(), e->val.p, sizeof(double) * e->nnz, hipMemcpyDeviceToHost, s));
+  NRT_HIP(hipMemcpyAsync(type.data(), e->hh_type.p, sizeof(int32_t) * H, hipMemcpyDeviceToHost, s));
+  NRT_HIP(hipStreamSynchronize(s));
+  for (int hh = 0; hh < H; hh++)  // an HH ghost or sealed end gates without a row of its own
+    if (type[hh] == RT_OTHER || type[hh] == RT_TERM) return false;
+  // matrix, c_m dx / dT, K dx; the state
+  std::vector<double> mat(5 * (size_t)N, 0.0), x(p.V0), inp;
+  for (int i = 0; i < N; i++) {
+    for (int k = rowptr[i]; k < rowptr[i + 1]; k++) {
+      if (col[k] < i - 1 || col[k] > i + 1) return false;
+      mat[(size_t)(col[k] - i + 1) * N + i] = val[k];
+    }
+    mat[3 * (size_t)N + i] = cmdx[i] / p.dT;
+    mat[4 * (size_t)N + i] = kdx[i];
+    if (p.input[i] != 0.0) {
+      if (inp.empty()) inp.assign(N, 0.0);
+      inp[i] = p.input[i];
+    }
+  }
+  std::vector<int32_t> i32(woff);
+  for (const auto* g : {&p.m, &p.h, &p.n})
+    for (const auto& [row, k] : rows) x.push_back((*g)[k]);
+  for (const auto& [row, k] : rows) i32.push_back(row);
+  for (const auto& [row, k] : rows) i32.push_back(k);
+  e->x.upload(x, s);
+  e->rx2.upload(x, s);
+  e->rcdt.upload(mat, s);
+  if (!inp.empty()) e->rinp.upload(inp, s);
+  e->rinf32.upload(i32, s);
+  const size_t words = 2 * (size_t)W * 7 * 2;
+  e->rll.alloc(words);
+  NRT_HIP(hipMemsetAsync(e->rll.p, 0, sizeof(unsigned long long) * words, s));
+  NRT_HIP(hipStreamSynchronize(s));  // the host arrays end here
+  const double* at = e->rcdt.p;
+  const int32_t* ii = e->rinf32.p;
+  e->cdev = ChainDev{N, W, C, H, at, at + N, at + 2 * (size_t)N, at + 3 * (size_t)N,
+                     at + 4 * (size_t)N, e->rinp.p, ii, ii + W + 1, ii + W + 1 + H, nullptr,
+                     nullptr, e->rll.p};
+  e->rdev = ResDev{};
+  e->rdev.G = W;
+  e->rdev.x = e->x.p;
+  e->rdev.xo = e->rx2.p;
+  e->chain = e->resident = true;
+  e->ns0 = N;
+  e->nblocks = W;
+  e->threads = 64;
+  e->rowptr.release();
+  e->col.release();
+  return true;
+}
+
 Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threads) {
   hipStream_t s = hnd->stream;
   const int N = p.N, H = p.H;
@@ -2344,7 +2433,9 @@ Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threa
           NRT_REQUIRE(hcol[k] <= i || par[hcol[k]] == i, NRT_ERR_TOPOLOGY,
                       "tree solve: row " + std::to_string(i) + " couples to row " +
                           std::to_string(hcol[k]) + ", which does not couple back");
-      if (e->method == 1 && resident_create(hnd, e, p, par, hrp, hcol, cmdx, kdx, batch_threads > 0)) {
+      if (e->method == 1 &&
+          (resident_create(hnd, e, p, par, hrp, hcol, cmdx, kdx, batch_threads > 0) ||
+           (batch_threads == 0 && chain_create(hnd, e, p, par, hrp, hcol, cmdx, kdx)))) {
         // (everything is set up: rows, plan, launch form)
       } else {
       // Workgroups: every reduction level costs a grid barrier (an L2 write-back), so
@@ -2686,7 +2777,7 @@ static ImpDev imp_dev(nrt_handle* hnd) {
 // level-0 slot for the tree solve.
 static int32_t probe_index(const Implicit* e, int32_t elem, int64_t interval) {
   if (interval < 0 || elem < 0 || elem >= e->N) return 0;  // no probe: never read
-  return e->method == 0 ? elem : e->resident ? e->rslot[elem] : e->plan_h.slot0[elem];
+  return e->method == 0 ? elem : e->resident ? (e->chain ? elem : e->rslot[elem]) : e->plan_h.slot0[elem];
 }
 
 template <class T>
@@ -2775,6 +2866,13 @@ static int launch_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_
     const ResRun q{first, num, gl0, e->rtag, trace_dev,
                    retried ? std::min(d.spin_limit, 20000ull) : d.spin_limit};
     e->rtag += (unsigned)num;
+    if (e->chain) {
+      ChainDev c = e->cdev;
+      c.x = e->rdev.x;
+      c.xo = e->rdev.xo;
+      chain_launch(d, c, q, hnd->stream);
+      return NRT_OK;
+    }
     resident_launch(d, e->rdev, q, hnd->stream);
     return NRT_OK;
   }

@@ -94,6 +94,13 @@ __device__ __forceinline__ void wave_sum_comp(float& s, float& c) {
   c = cc;
 }
 
+// 1 / x to about an ulp (the hardware's estimate and two Newton steps).
+__device__ __forceinline__ double rcp_newton(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
 // Sum of NV values over the block (blockDim.x a multiple of 64, <= 1024); the
 // result is returned to every thread. lds must hold NV*16 doubles.
 template <int NV>

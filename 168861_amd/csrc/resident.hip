@@ -13,20 +13,6 @@ __device__ __forceinline__ double lane_get(double x, int byte_lane) {
   return __hiloint2double(hi, lo);
 }
 
-// Diagonal of the HH row q for the membrane term W (hh_row_refresh without the row's
-// values in memory).
-__device__ __forceinline__ double hh_row_diag(const HHRow& q, double W) {
-  const double betaMe = -(W * q.dxv) + q.inv_rdx;
-  const double beta = q.c_dt + betaMe + q.betaR;
-  switch (q.type) {
-    case RT_NEXT_TERM: return beta + -q.betaR;
-    case RT_BRANCH: return beta + q.betaL;
-    case RT_FIRST_NORMAL: return q.alpha + beta;
-    case RT_FIRST_BRANCH: return q.alpha + beta + q.betaL;
-    default: return beta;
-  }
-}
-
 // The dynamic rows' state in LDS (read by the service wave once a step: kept in its
 // registers it would cost every wave of the workgroup the same registers).
 struct DynRow {
@@ -64,12 +50,6 @@ __device__ __forceinline__ void dyn_load(const ImpDev& d, const ResDev& r, int j
   }
   y.parent = f[4] == 0xFFFF ? -1 : f[4];
   *out = y;
-}
-// 1 / x to about an ulp (the hardware's estimate and two Newton steps).
-__device__ __forceinline__ double rcp_newton(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.0), r, r);
-  return fma(fma(-x, r, 1.0), r, r);
 }
 // The service wave, eight lanes a dynamic row: gating (hh_gate_step; lanes 0..5 of a row
 // evaluate one rate function each, so it costs one exponential's latency instead of

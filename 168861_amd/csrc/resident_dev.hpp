@@ -5,6 +5,20 @@
 
 namespace nrt {
 
+// Diagonal of the HH row q for the membrane term W (hh_row_refresh without the row's
+// values in memory).
+__device__ __forceinline__ double hh_row_diag(const HHRow& q, double W) {
+  const double betaMe = -(W * q.dxv) + q.inv_rdx;
+  const double beta = q.c_dt + betaMe + q.betaR;
+  switch (q.type) {
+    case RT_NEXT_TERM: return beta + -q.betaR;
+    case RT_BRANCH: return beta + q.betaL;
+    case RT_FIRST_NORMAL: return q.alpha + beta;
+    case RT_FIRST_BRANCH: return q.alpha + beta + q.betaL;
+    default: return beta;
+  }
+}
+
 struct ResDev {
   int G, T, nd, nt, npub, nth, top_narrow, rounds, owner, has_input;
   // rows, slot order
