@@ -638,7 +638,8 @@ const double* explicit_slot_v(nrt_handle* h, long long done) {
 }
 
 int64_t explicit_device_bytes(const Explicit* e) {
-  return (int64_t)e->N * (8 * 6 + 4) + (int64_t)e->R * 40 + (int64_t)e->H * 8 * 13;
+  return (int64_t)e->N * (8 * 6 + 4) + (int64_t)e->R * 40 + (int64_t)e->H * 8 * 13 +
+         (int64_t)(e->tunit.n + e->tdyn.n) * 40 + (int64_t)e->ll.n * 8;
 }
 
 }  // namespace nrt

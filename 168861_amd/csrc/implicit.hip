@@ -105,6 +105,7 @@ struct Implicit {
   DBuf<int32_t> rslot_dev;  // rslot on the device (snapshots)
   unsigned rtag = 0;  // tag of the last step launched
   int64_t rsteps = 0;
+  HostWord rword;     // several workgroups: a launch gave up
   unsigned rerr = 0;  // the last launch gave up
   std::vector<int32_t> rslot;  // element -> index in x (empty: the element itself)
   // unbranched neurites (chain.hip; resident is set too)
@@ -2206,6 +2207,7 @@ static bool resident_create(nrt_handle* hnd, Implicit* e, const HostProblem& p,
   r.ll = e->rll.p;
   NRT_HIP(hipStreamSynchronize(s));  // the host arrays end here
   e->resident = true;
+  if (!in_batch && P.G > 1) e->rword.take();
   e->rslot = std::move(P.slot);
   e->ns0 = (int)n0;
   e->nblocks = P.G;
@@ -2292,6 +2294,7 @@ static bool chain_create(nrt_handle* hnd, Implicit* e, const HostProblem& p,
   e->rdev.x = e->x.p;
   e->rdev.xo = e->rx2.p;
   e->chain = e->resident = true;
+  if (W > 1) e->rword.take();
   e->ns0 = N;
   e->nblocks = W;
   e->threads = 64;
@@ -2866,6 +2869,7 @@ static int launch_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_
     const ResRun q{first, num, gl0, e->rtag, trace_dev,
                    retried ? std::min(d.spin_limit, 20000ull) : d.spin_limit};
     e->rtag += (unsigned)num;
+    if (e->rword.p) d.err = e->rword.p;
     if (e->chain) {
       ChainDev c = e->cdev;
       c.x = e->rdev.x;
@@ -3075,12 +3079,10 @@ static void run_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_t 
       return;
     }
     if (e->rdev.G > 1) {
-      unsigned err = 0;
-      NRT_HIP(hipMemcpyAsync(&err, e->bar.p + 2, sizeof(unsigned), hipMemcpyDeviceToHost,
-                             hnd->stream));
       NRT_HIP(hipStreamSynchronize(hnd->stream));
+      const unsigned err = e->rword.get();
+      e->rword.clear();
       if (err && std::chrono::steady_clock::now() < until) {
-        reset_barrier(e, hnd->stream);
         // (handles of different processes wait differently: their addresses differ)
         std::this_thread::sleep_for(std::chrono::microseconds(
             100 * std::min(attempt + 1, 50) + (int)((uint32_t)((uintptr_t)e >> 6) * 2654435761u >> 22)));

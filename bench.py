@@ -58,6 +58,13 @@ def tree_bytes(N, H, nnz, steps, solves, vbytes):
     return steps * per_step + solves * per_solve + (solves + steps) * per_resid
 
 
+def resident_bytes(N, H, launches):
+    """Rows kept in registers for a launch (k_resident*, k_chain): V read and written, two
+    coefficients of the row's equation and three of its right-hand side, once per launch
+    whatever its steps; 120 B of gates (read and written) and parameters per HH row."""
+    return launches * (56 * N + 120 * H)
+
+
 def bicgstab_bytes(N, H, nnz, steps, iters):
     """Per step 144 B per HH element + 40 B per element (update phase); per
     BiCGSTAB iteration 2 SpMV (12 nnz + 4 (N+1) + 16 N) + 21 vector passes of 8 N."""
@@ -283,8 +290,13 @@ def sweep_leg(nh, wl, orc, a, info):
         nb = sum(tree_bytes(p.N, p.H, nz, a.steps, sv, vb)
                  for p, nz, sv in zip(imp, r["nnz"], r["solves"]))
         # one k_batch_tree launch per size class, concurrent: the roofline is the
-        # group's (all classes' bytes over the time from the first start to the last end)
+        # group's (all classes' bytes over the time from the first start to the last end);
+        # FP64 slots planned without a chunk length keep their rows in registers
         kern = f"k_batch_tree<{'double' if vb == 8 else 'float'},*>"
+        shapes = (r["tune"] or {}).get("classes", {}).values()
+        if vb == 8 and all(c["chunk"] == "auto" for c in shapes):
+            kern = "k_resident_batch"
+            nb = resident_bytes(Ntot, H, r["launches"])
         rec = {"compartment_steps_per_s": r["compartment_steps"] / r["wall_s"],
                "ms_per_step": r["wall_s"] / a.steps * 1e3, "status": r["status"],
                "solves_per_step": sum(r["solves"]) / len(imp) / a.steps,
@@ -309,11 +321,12 @@ def sweep_leg(nh, wl, orc, a, info):
     ex_snap = {i: b.snapshot(ids[i]) for i in sample[::4]}
     ex_done = b.info(ids[sample[0]])["steps_done"]
     b.close()
-    nb = explicit_bytes(sum(p.N for p in exp_), sum(p.H for p in exp_)) * a.steps
+    # (elements in registers for a launch: what a step needs of memory, once per launch)
+    nb = explicit_bytes(sum(p.N for p in exp_), sum(p.H for p in exp_)) * r["launches"]
     rec = {"compartment_steps_per_s": r["compartment_steps"] / r["wall_s"],
            "ms_per_step": r["wall_s"] / a.steps * 1e3,
-           "roofline": roofline(nb, r["kernel_ms"], "k_explicit_batch", a.steps,
-                                measured_traffic("k_explicit_batch", wname, 1))}
+           "roofline": roofline(nb, r["kernel_ms"], "k_explicit_tree_batch", r["launches"],
+                                measured_traffic("k_explicit_tree_batch", wname, per_launch))}
     if orc is not None:
         errs = []
         for i, v in ex_snap.items():
@@ -461,9 +474,9 @@ def config1_leg(nh, wl, orc, a):
                "ms_per_step": wall / steps * 1e3, "finite": bool(np.all(np.isfinite(v))),
                "max_abs_V_mV": float(np.max(np.abs(v))) * 1e3}
         if st["kernel_ms"] > 0:
-            nb = explicit_bytes(prob.N, prob.H) * steps
             launches = st["kernel_launches"]
-            kern = "k_explicit_resident" if launches == 1 else "k_explicit_fp64"
+            nb = explicit_bytes(prob.N, prob.H) * launches  # (one launch: in registers)
+            kern = "k_explicit_cable" if launches == 1 else "k_explicit_fp64"
             rec["roofline"] = roofline(nb, st["kernel_ms"], kern, launches)
         if orc is not None:
             ex = orc.Explicit(prob)
@@ -500,6 +513,9 @@ def implicit_forms(nh, prob, forms, a0, a1, orc):
         if kr == nh.DIRECT:
             nb = tree_bytes(prob.N, prob.H, st["matrix_nnz"], steps, inner, vb)
             kern = nh.TREE_KERNELS[st["tree_form"]].format(T="double" if vb == 8 else "float")
+            if st["tree_form"] == nh.TREE_RESIDENT:
+                nb = resident_bytes(prob.N, prob.H, 1)
+                kern = "k_chain" if prob.H > 8 else kern
         elif kr == nh.GMRES:
             cycles = st["refine_sweeps"] if vb == 4 else st["restarts"] + steps
             nb = gmres_bytes(prob.N, prob.H, st["matrix_nnz"], steps, inner, cycles, vb)
