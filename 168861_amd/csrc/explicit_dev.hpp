@@ -55,7 +55,7 @@ struct Explicit {
   unsigned tag = 0;
   // branching neurites with their elements in registers (explicit_tree.hip); they use
   // the second gates and the exchange of the fields above
-  int tree_groups = 0, tree_T = 0, tree_slots = 0;
+  int tree_groups = 0, tree_T = 0, tree_slots = 0, tree_every = 0;
   DBuf<ExUnit> tunit;
   DBuf<ExDynUnit> tdyn;
   HHDev hd() {

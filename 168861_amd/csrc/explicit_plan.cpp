@@ -7,12 +7,13 @@
 
 namespace nrt {
 
-bool build_explicit_plan(const HostProblem& p, int T, ExPlanHost& P, std::string& why) {
+bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, std::string& why) {
   constexpr int C = kExC;
   P = ExPlanHost();
   const int N = p.N;
   P.N = N;
   P.T = T;
+  P.every = every;
   auto no = [&](const char* w) {
     why = w;
     return false;
@@ -110,7 +111,7 @@ bool build_explicit_plan(const HostProblem& p, int T, ExPlanHost& P, std::string
       fresh.clear();
       todo.clear();
       auto see = [&](int w, int dist, int from, bool from_up) {
-        if (w >= 0 && dist <= kExEvery) todo.push_back({w, dist, from, from_up});
+        if (w >= 0 && dist <= every) todo.push_back({w, dist, from, from_up});
       };
       see(node[s].up, 1, s, false);
       see(node[s].right, 1, s, true);
@@ -221,7 +222,8 @@ extern "C" int nrt_test_explicit_tree_host(const nrt_problem* np, int T, int ste
   }
   ExPlanHost P;
   std::string w;
-  const bool ok = build_explicit_plan(p, T, P, w);
+  const bool ok = build_explicit_plan(p, T, kExEvery, P, w) ||
+                  build_explicit_plan(p, T, kExEveryDense, P, w);
   if (why && why_len > 0) {
     std::strncpy(why, w.c_str(), (size_t)why_len - 1);
     why[why_len - 1] = 0;
@@ -244,7 +246,7 @@ extern "C" int nrt_test_explicit_tree_host(const nrt_problem* np, int T, int ste
   auto rdx = [&](int j) { return p.r_a[j] * p.dx[j]; };
   for (int st = 1; st <= steps; st++) {
     const bool active = st >= a0 && st <= a1;
-    if (st > 1 && (st - 1) % kExEvery == 0)
+    if (st > 1 && (st - 1) % P.every == 0)
       for (int put = 1; put >= 0; put--) {
         for (int i = 0; i < G * T; i++) {
           const ExUnit& u = P.unit[i];
@@ -346,7 +348,7 @@ extern "C" int nrt_test_explicit_tree_host(const nrt_problem* np, int T, int ste
     V[u.elem] = D[i].v;
     if (u.flags & kExUGhost) V[0] = v0[i / kExDyn];
   }
-  const int32_t out[4] = {G, P.T, P.slots, P.units};
+  const int32_t out[5] = {G, P.T, P.slots, P.units, P.every};
   if (info) std::memcpy(info, out, sizeof(out));
   return 0;
 }

@@ -7,7 +7,7 @@
 // neighbours' potentials from LDS (double buffered) and stores its two ends, and a step
 // is one barrier. What bounds it: the FP64 operations, about 13 an element and step
 // (8 elements a thread; 2 waves a SIMD at kExT units), the barrier, and the exchange
-// between groups, a round trip through memory, once in kExEvery steps.
+// between groups, a round trip through memory, once in 16 steps.
 //
 // Every operation is explicit_element's, operand for operand (an axial term of an element
 // and its mother is computed once: it enters the two with opposite signs, which loses
@@ -21,7 +21,7 @@
 namespace nrt {
 
 struct ExTreeDev {
-  int N, G, T, slots;
+  int N, G, T, slots, every;
   const ExUnit* unit;
   const ExDynUnit* dyn;
   double* V[2];
@@ -91,7 +91,7 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
   }
   const bool service = tid >= T && tid < T + kWave;
   // what an exchange needs, and when
-  const int every = d.slots > 0 ? kExEvery : INT_MAX;
+  const int every = pinned_s(d.slots > 0 ? d.every : INT_MAX);
   auto words = [&](unsigned tag, int slot) {
     return as_global(d.ll) + ((size_t)(tag & 1) * d.slots + slot) * kExSlotVals * 2;
   };
@@ -428,7 +428,8 @@ void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_ba
   const auto plan = [&](int T, int most) {
     // (strands of some 50 elements and halos: 4 to 6% more units than N / kExC)
     if (p.N / kExC * 1.03 > (double)most * T) return;
-    if (build_explicit_plan(p, T, P, why)) fits = P.G <= most;
+    for (int every : {kExEvery, kExEveryDense})
+      if (!fits && build_explicit_plan(p, T, every, P, why)) fits = P.G <= most;
   };
   plan(kExTBatch, cap);
   if (!in_batch && !fits) plan(kExTLarge, cap);
@@ -437,6 +438,7 @@ void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_ba
   e->tree_groups = P.G;
   e->tree_T = P.T;
   e->tree_slots = P.slots;
+  e->tree_every = P.every;
   e->tunit.upload(P.unit, hnd->stream);
   e->tdyn.upload(P.dyn, hnd->stream);
   e->m2.alloc(p.H);
@@ -452,7 +454,7 @@ void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_ba
 
 static ExTreeDev tree_dev(Explicit* e, int from, unsigned* err, long long a0, long long a1,
                           long long interval, int trace_elem) {
-  return {e->N, e->tree_groups, e->tree_T, e->tree_slots, e->tunit.p, e->tdyn.p,
+  return {e->N, e->tree_groups, e->tree_T, e->tree_slots, e->tree_every, e->tunit.p, e->tdyn.p,
           {e->V[from].p, e->V[1 - from].p}, e->coefA.p, e->rdx.p, e->wdx.p, e->kdx.p, e->hd(),
           e->m2.p, e->h2.p, e->n2.p, e->dt_ms, e->ll.p, err, a0, a1, interval, trace_elem};
 }
@@ -469,7 +471,7 @@ bool tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t 
       [&](unsigned long long first_limit, unsigned long long limit) {
         const ExTreeDev d = tree_dev(e, e->cur, e->err.p, a0, a1, interval, trace_elem);
         ExTreeRun q{0, (long long)first, (long long)num, 0, trace, e->tag, first_limit, limit};
-        e->tag += (unsigned)(num / kExEvery + 2);
+        e->tag += (unsigned)(num / e->tree_every + 2);
         hipLaunchKernelGGL(k_explicit_tree, dim3(e->tree_groups), dim3(e->tree_T + kWave), 0,
                            hnd->stream, d, q);
       },
@@ -497,7 +499,7 @@ void explicit_tree_work(nrt_handle* h, long long done, long long steps, void* ou
   const ExTreeWork w{done, steps, e->cur, e->tag};
   memcpy(out, &w, sizeof(w));
   if (steps <= 0) return;
-  e->tag += (unsigned)(steps / kExEvery + 2);
+  e->tag += (unsigned)(steps / e->tree_every + 2);
   e->cur = 1 - e->cur;
 }
 // A launch that timed out: the potentials before it are the current ones again.

@@ -5,10 +5,12 @@
 // thread's; a chain is cut from its end, so its first unit may begin with unused
 // places. At most kExDyn HH elements stand outside the units, each with lanes of its own.
 // A group (workgroup) owns consecutive units and computes, besides, every unit with an
-// element at most kExEvery elements away from one that it owns (its halo): without the
+// element at most `every` elements away from one that it owns (its halo): without the
 // neighbours that are missing there, the halo's values become wrong from its outside, one
-// element a step, and reach no owned element within kExEvery steps, after which the
-// halo's values are fetched from their owners.
+// element a step, and reach no owned element within `every` steps, after which the
+// halo's values are fetched from their owners. `every` is kExEvery, or kExEveryDense where
+// a halo of that width would not fit (branches a few elements apart: the halo doubles at
+// each).
 #pragma once
 #include <cstdint>
 #include <string>
@@ -20,7 +22,7 @@ namespace nrt {
 constexpr int kExC = 8;      // elements per unit
 constexpr int kExT = 512;    // most units (owned and halo) per group
 constexpr int kExDyn = 8;    // most HH elements
-constexpr int kExEvery = 16;  // steps between exchanges
+constexpr int kExEvery = 16, kExEveryDense = 4;  // steps between exchanges
 
 // Unit flags; the number of unused places is in bits 0..2, the place of the element with
 // a stimulus (one at most) in bits 8..10.
@@ -52,12 +54,12 @@ static_assert(sizeof(ExUnit) == 40 && sizeof(ExDynUnit) == 40, "plan records");
 constexpr int kExSlotVals = kExC;  // doubles of an exchange slot (V; of an HH element V, m, h, n)
 
 struct ExPlanHost {
-  int N = 0, G = 0, T = 0, slots = 0, units = 0;
+  int N = 0, G = 0, T = 0, slots = 0, units = 0, every = 0;
   std::vector<ExUnit> unit;    // [G * T]
   std::vector<ExDynUnit> dyn;  // [G * kExDyn]
 };
 
 // Groups of at most T <= kExT units (one of as many as needed, where that is enough).
-bool build_explicit_plan(const HostProblem& p, int T, ExPlanHost& P, std::string& why);
+bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, std::string& why);
 
 }  // namespace nrt

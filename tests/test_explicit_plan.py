@@ -17,11 +17,11 @@ def tree_host(p, T, steps, a0, a1):
     f = nh.lib().nrt_test_explicit_tree_host
     f.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_double),
                   C.POINTER(C.c_int32), C.c_char_p, C.c_int]
-    v, info, why = np.full(p.N, np.nan), np.zeros(4, np.int32), C.create_string_buffer(100)
+    v, info, why = np.full(p.N, np.nan), np.zeros(5, np.int32), C.create_string_buffer(100)
     s = p.struct()
     st = f(C.addressof(s), T, steps, a0, a1, v.ctypes.data_as(C.POINTER(C.c_double)),
            info.ctypes.data_as(C.POINTER(C.c_int32)), why, 100)
-    return (v, dict(zip(("G", "T", "slots", "units"), info.tolist()))) if st == 0 else \
+    return (v, dict(zip(("G", "T", "slots", "units", "every"), info.tolist()))) if st == 0 else \
         why.value.decode()
 
 
@@ -50,6 +50,19 @@ def test_trees_bitwise(depth, T, hh, orc):
     assert (got[1]["G"] > 1) == (got[1]["units"] > T) == (got[1]["slots"] > 0)
     ref = orc.Explicit(p)
     ref.run(1, 40, 5, 25)
+    assert np.array_equal(got[0], ref.snapshot())
+
+
+@pytest.mark.parametrize("tree,T", [(0, 192), (0, 64), (240, 64), (480, 192)])
+def test_dense_branching_bitwise(tree, T, orc):
+    """Segments of a few elements: a halo of 16 elements does not fit, one of 4 does."""
+    geom = wl.sweep_tree(tree)[0]
+    s, bufs, H = _setup(orc, geom)
+    p = _problem(geom, s, bufs, H, 0.8 * float(s.dT_crit))
+    got = tree_host(p, T, 30, 1, 20)
+    assert not isinstance(got, str), got
+    ref = orc.Explicit(p)
+    ref.run(1, 30, 1, 20)
     assert np.array_equal(got[0], ref.snapshot())
 
 

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import neurite_hip as nh
+import workloads as wl
 from common import TOL_V, max_abs_diff
 from test_explicit_plan import _random_tree, tree_host
 
@@ -66,6 +67,23 @@ def test_runs_equal_single_steps(depth, hh, nrt, orc):
     ref.run(step, 1, step, step)
     ref.run(step + 1, 20, 1, 0)
     assert max_abs_diff(v, ref.snapshot()) <= TOL_V
+
+
+@pytest.mark.parametrize("tree", [0, 240, 480, 4000])
+def test_dense_branching(tree, nrt):
+    """Segments of a few elements: exchanges every 4 steps (a run ends within, at and after
+    one), alone and in a batch."""
+    p, _ = nrt.setup(wl.sweep_tree(tree)[0], dT=None, dt_factor=0.8)
+    with nrt.Solver(p, kind=nh.EXPLICIT) as s, nrt.Batch(kind=nh.EXPLICIT) as b:
+        slot = b.add(p, 1000, 1, 20)
+        step = 0
+        for c in (3, 4, 5, 30):
+            s.run(step + 1, c, 1, 20)
+            b.step(c)
+            assert b.stats()["launches"] > 0 and s.stats()["kernel_launches"] == 1
+            step += c
+        v = _stepped(nrt, p, step, 1, 20)
+        assert np.array_equal(s.snapshot(), v) and np.array_equal(b.snapshot(slot), v)
 
 
 def test_batch_slots(nrt, orc):
