@@ -1,8 +1,8 @@
 // Batches of independent neurites (the nrt_batch_* entry points). Each slot is a
 // complete solver state (a handle without a stream of its own); the batch keeps a
 // device table of slot descriptors that is rebuilt only when membership changes,
-// and advances all slots with one launch per call (implicit, persistent over the
-// k steps) or one graph of k steps (explicit).
+// and advances all slots with one launch per call (persistent over the k steps) or,
+// for explicit slots whose elements cannot stay in registers, one graph of k steps.
 #include <algorithm>
 #include <chrono>
 #include <climits>
@@ -86,7 +86,6 @@ constexpr int64_t kAdmissionReserve = 512ll << 20;  // left free for the runtime
 // in a launch of their own while they fill the device: a workgroup of the large ones'
 // size would leave two thirds of its waves idle.
 constexpr int kResSmallT = 192;
-constexpr int kExSmallFill = 1024;  // explicit slots of that size that fill the device
 struct ResStep {  // ResWork of resident_dev.hpp
   long long done, steps;
 };
@@ -251,9 +250,9 @@ struct nrt_batch {
     dirty = false;
   }
 
-  // Takes the slots with a resident tree solve out of `order`. Those of at most
-  // kResSmallT unit threads a workgroup get a launch of their own while they fill the
-  // device (as size classes do); else all share one.
+  // Takes the slots whose rows stay in registers out of `order`. Those of at most
+  // kResSmallT unit threads a workgroup (explicit ones all are) get a launch of their own
+  // while they fill the device (as size classes do); else all share one.
   void rebuild_resident() {
     for (ResClass& c : res) c = ResClass();
     std::vector<int> rest;
@@ -273,8 +272,7 @@ struct nrt_batch {
     }
     order.swap(rest);
     if (!res[0].ids.empty() && !res[1].ids.empty() &&
-        (int)res[1].ids.size() <
-            (is_implicit() ? resident_capacity(device, res[1].T, res[1].lds) : kExSmallFill) / 2) {
+        (int)res[1].ids.size() < resident_capacity(device, res[1].T, res[1].lds) / 2) {
       res[0].ids.insert(res[0].ids.end(), res[1].ids.begin(), res[1].ids.end());
       res[0].lds = std::max(res[0].lds, res[1].lds);
       res[0].maxG = std::max(res[0].maxG, res[1].maxG);

@@ -1,4 +1,6 @@
-// Explicit (FTCS + forward-Euler HH) step, FP64 plain form, one fused kernel.
+// Explicit (FTCS + forward-Euler HH) step, FP64 plain form, one fused kernel that goes
+// over memory (single steps, batch slots and runs that explicit_cable.hip and
+// explicit_tree.hip do not take).
 //
 // Semantics follow the reference CPU solver, the general-topology one
 // (solverEx-cpu.cpp:45-123 with hhRate_Const coupling.cpp:25-48); the reference
@@ -226,8 +228,8 @@ __global__ __launch_bounds__(256) void k_explicit_fp64(
   explicit_element(j, N, Vo, Vn, coefA, rdx, wdx, kdx, code, recs, hd, dt_ms, active != 0);
 }
 
-// Whole runs of a small neurite in one workgroup: both potentials live in LDS
-// for the launch and the steps are separated by workgroup barriers instead of
+// Whole runs of a small neurite in one workgroup (trees with many HH elements, and one
+// or two steps of any): both potentials live in LDS for the launch and the steps are separated by workgroup barriers instead of
 // kernel launches (a launch per step costs more than a thousand elements' work).
 // The element update is explicit_element's, operand for operand.
 constexpr int kResBlock = 1024;

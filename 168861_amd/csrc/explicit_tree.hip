@@ -7,7 +7,10 @@
 // neighbours' potentials from LDS (double buffered) and stores its two ends, and a step
 // is one barrier. What bounds it: the FP64 operations, about 13 an element and step
 // (8 elements a thread; 2 waves a SIMD at kExT units), the barrier, and the exchange
-// between groups, a round trip through memory, once in 16 steps.
+// between groups, a round trip through memory, once in 16 steps. Measured, us a step
+// before (small neurites from LDS and L2 in one workgroup, others a launch a step) and
+// here: 700 elements 2.3 and 0.6, 3,001 3.8 and 0.65, 30,000 4.2 and 0.7, 300,000 5.7 and
+// 0.8, 902,037 10.7 and 1.5; a batch of 512 trees (5.5 M elements) 55 and 8.
 //
 // Every operation is explicit_element's, operand for operand (an axial term of an element
 // and its mother is computed once: it enters the two with opposite signs, which loses
@@ -44,7 +47,11 @@ struct ExTreeRun {
   unsigned long long first_limit, limit;
 };
 
-constexpr int kExTBatch = 192;  // most units per group in a batch
+// Most units per group, as long as the groups are at most the CUs: with the HH elements' wave
+// four waves, one a SIMD (0.68 us a step for 30,000 elements; with 256 units, two waves on
+// one SIMD, 0.97) and three workgroups a CU in a batch (five-wave ones only one: 100 steps
+// of 512 trees 1.5 ms, with 192 units 1.05).
+constexpr int kExTBatch = 192;
 constexpr int kExTBlock = kExT + kWave;
 
 // What the loop over the steps needs of the records stays in scalar registers: a batch's
@@ -431,6 +438,7 @@ void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_ba
     for (int every : {kExEvery, kExEveryDense})
       if (!fits && build_explicit_plan(p, T, every, P, why)) fits = P.G <= most;
   };
+  // (larger groups where there are not CUs enough: seven or eight waves of units)
   plan(kExTBatch, cap);
   if (!in_batch && !fits) plan(kExTLarge, cap);
   if (!in_batch && !fits) plan(kExT, cap);

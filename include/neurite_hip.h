@@ -232,7 +232,8 @@ typedef struct nrt_stats {
 #define NRT_TREE_GRID       1  /* level-synchronous grid (a barrier per level)   */
 #define NRT_TREE_LOCAL      2  /* local mode, levels in global memory            */
 #define NRT_TREE_LOCAL_LDS  3  /* local mode, each group's levels in its LDS     */
-#define NRT_TREE_RESIDENT   4  /* rows resident in registers (few rows change)   */
+#define NRT_TREE_RESIDENT   4  /* rows resident in registers (few rows change,
+                                  or an unbranched neurite)                      */
 
 typedef struct nrt_handle nrt_handle;
 
@@ -300,8 +301,10 @@ int nrt_sync(nrt_handle* h);
  *     slots of each size class (< 4,096 rows, < 16,384, the rest) run as a launch
  *     of their own, concurrently, while every class fills at least half the
  *     device, else all in one launch;
- *   explicit: one thread per element over all slots, one launch per step, the k
- *     steps of a call captured once as a HIP graph and replayed.
+ *   explicit: the k steps of a call in one launch with every element in registers
+ *     (at most eight HH elements on a tree or cable); other slots one thread per
+ *     element, one launch per step, the k steps captured once as a HIP graph and
+ *     replayed.
  * Slots keep their whole state on the device and join or leave between calls
  * (continuous batching). A slot counts its own steps from 1: its stimulus is on
  * for steps a0..a1 and it completes after num_steps. Probe traces follow
