@@ -385,7 +385,8 @@ Explicit* explicit_create(nrt_handle* hnd, const HostProblem& p, bool in_batch) 
     e->rest.upload(p.rest, s);
     e->hdx.upload(hdx, s);
     cable_prepare(hnd, e, p, in_batch);
-    if (e->cable_groups == 0) tree_prepare(hnd, e, p, in_batch);
+    ExPlanHost plan;
+    if (e->cable_groups == 0) tree_prepare(hnd, e, p, in_batch, plan);
     NRT_HIP(hipStreamSynchronize(s));
   } catch (...) {
     delete e;

@@ -137,7 +137,8 @@ bool cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t
                int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0, hipEvent_t t1);
 
 // explicit_tree.hip
-void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_batch);
+void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_batch,
+                  ExPlanHost& P);
 bool tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
               int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0, hipEvent_t t1);
 

@@ -19,27 +19,38 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
     return false;
   };
   if (N < 4 || p.T < 1 || p.terminals[0] != 0) return no("first terminal");
-  std::vector<uint8_t> term(N, 0);
+  std::vector<uint8_t> mark(N + 1, 0);  // 1: sealed end, 2: HH element
+  struct Bit {
+    const uint8_t* m;
+    uint8_t b;
+    bool operator[](int j) const { return m[j] & b; }
+  };
+  const Bit term{mark.data(), 1}, hh{mark.data(), 2};
   for (int k = 0; k < p.T; k++) {
     if (k > 0 && p.terminals[k] == 0) return no("first terminal twice");
-    term[p.terminals[k]] = 1;
+    mark[p.terminals[k]] = 1;
   }
   if (!term[N - 1]) return no("last element is no sealed end");
   if (p.H > kExDyn) return no("too many HH elements");
-  std::vector<int32_t> hh(N, -1);
   for (int i = 0; i < p.H; i++) {
     const int e = p.hh_elem[i];
-    if (term[e] || hh[e] >= 0) return no("HH element");
-    hh[e] = i;
+    if (mark[e]) return no("HH element");
+    mark[e] = 2;
   }
+  auto hh_index = [&](int e) {
+    return (int)(std::find(p.hh_elem.begin(), p.hh_elem.end(), e) - p.hh_elem.begin());
+  };
   if (p.mother[1] != 0) return no("element 1");
   // every computed element: its daughters name it as their mother, and the other way
   auto daughter = [&](int j, int d) { return d >= 1 && d < N && p.mother[d] == j; };
   for (int j = 1; j < N; j++) {
     const int m = p.mother[j];
+    if (j >= 2 && !(mark[j - 1] | mark[j] | mark[j + 1]) && m == j - 1 && p.dr[m] == j &&
+        !p.branching[j] && p.dr[j] == j + 1 && j + 1 < N && p.mother[j + 1] == j)
+      continue;  // (an element amid a strand: all of the below)
     if (term[j]) {
       // a sealed end: the next element after a passive, unbranched source
-      if (m != j - 1 || m < 1 || term[m] || hh[m] >= 0 || p.branching[m] || p.dr[m] != j)
+      if (m != j - 1 || m < 1 || term[m] || hh[m] || p.branching[m] || p.dr[m] != j)
         return no("sealed end");
       continue;
     }
@@ -51,7 +62,7 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
     if (p.branching[j]) {
       if (!daughter(j, p.dl[j]) || p.dl[j] == p.dr[j] || term[p.dl[j]] || term[p.dr[j]])
         return no("left daughter");
-    } else if (hh[j] >= 0 && term[p.dr[j]]) {
+    } else if (hh[j] && term[p.dr[j]]) {
       return no("sealed end of an HH element");
     }
   }
@@ -62,21 +73,21 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
   };
   std::vector<Node> node;
   node.reserve(N / C + N / 16 + 16);
-  std::vector<int32_t> node_of(N, -1);
+  std::vector<int32_t> node_of(N, -1);  // of first and last elements
   for (int j = 1; j < N;) {
-    if (hh[j] >= 0) {
+    if (hh[j]) {
       node_of[j] = (int)node.size();
-      node.push_back({j, 1, j, hh[j], -1, -1, -1});
+      node.push_back({j, 1, j, hh_index(j), -1, -1, -1});
       j++;
       continue;
     }
     int e = j;  // last element of the chain that starts at j
-    while (e + 1 < N && !term[e] && hh[e + 1] < 0 && p.mother[e + 1] == e && p.dr[e] == e + 1 &&
+    while (e + 1 < N && !term[e] && !hh[e + 1] && p.mother[e + 1] == e && p.dr[e] == e + 1 &&
            !p.branching[e])
       e++;
     int n = (e - j) % C + 1;
     for (int at = j; at <= e; at += n, n = C) {
-      for (int k = at; k < at + n; k++) node_of[k] = (int)node.size();
+      node_of[at] = node_of[at + n - 1] = (int)node.size();
       node.push_back({at, n, at + n - 1, -1, -1, -1, -1});
     }
     j = e + 1;
@@ -111,7 +122,8 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
       fresh.clear();
       todo.clear();
       auto see = [&](int w, int dist, int from, bool from_up) {
-        if (w >= 0 && dist <= every) todo.push_back({w, dist, from, from_up});
+        // (what lies beyond an owned node is nearer to that one, and there already)
+        if (w >= 0 && dist <= every && owner[w] != g) todo.push_back({w, dist, from, from_up});
       };
       see(node[s].up, 1, s, false);
       see(node[s].right, 1, s, true);

@@ -16,6 +16,7 @@
 // and its mother is computed once: it enters the two with opposite signs, which loses
 // nothing), so the results are those of the other kernels bit for bit.
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cstdlib>
 #include <cstring>
@@ -415,20 +416,26 @@ constexpr int kExTLarge = 448;
 // Groups that are sure to be resident at once: one a CU. (Where the registers allow two
 // of 256 unit threads, 477 of 512 did not all start.)
 int tree_capacity(int device, int T) {
+  static std::atomic<int> known{0};  // (device + 1) << 16 | CUs: asked for every slot of a batch
+  const int k = known.load(std::memory_order_relaxed);
+  if (k >> 16 == device + 1) return k & 0xFFFF;
   int cus = 0, per = 0;
   NRT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   NRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_explicit_tree,
                                                        T + kWave, 0));
-  return per > 0 ? cus : 0;
+  if (per == 0) cus = 0;
+  known.store((device + 1) << 16 | cus, std::memory_order_relaxed);
+  return cus;
 }
 }  // namespace
 
-void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_batch) {
+// (P: the plan is uploaded from it until the stream is waited for)
+void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_batch,
+                  ExPlanHost& P) {
   // (a run of an unbranched neurite is the cable kernel's or specified as a launch a step)
   bool branching = in_batch;
   for (int j = 1; j < p.N - 1 && !branching; j++) branching = p.branching[j] != 0;
   if (!branching) return;
-  ExPlanHost P;
   std::string why;
   bool fits = false;
   const int cap = tree_capacity(hnd->device, kExT);
@@ -457,7 +464,6 @@ void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_ba
     e->ll.alloc((size_t)2 * P.slots * kExSlotVals * 2);
     NRT_HIP(hipMemsetAsync(e->ll.p, 0, sizeof(unsigned long long) * e->ll.n, hnd->stream));
   }
-  NRT_HIP(hipStreamSynchronize(hnd->stream));  // (the plan is read until here)
 }
 
 static ExTreeDev tree_dev(Explicit* e, int from, unsigned* err, long long a0, long long a1,
