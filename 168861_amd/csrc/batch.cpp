@@ -373,7 +373,8 @@ struct nrt_batch {
   // elem_budget > 0 (implicit only), max(1, min(kmax, elem_budget / N)) each, so
   // that one launch takes about the same time whatever the sizes and small
   // slots do not wait on large ones. Slots added before finish() join after it.
-  void launch(long long k, long long elem_budget = 0, long long kmax = 0) {
+  // shared: the caller holds the device's CUs for this launch (device_share).
+  void launch(long long k, long long elem_budget = 0, long long kmax = 0, bool shared = false) {
     NRT_REQUIRE(k >= 0, NRT_ERR_INVALID, "k < 0");
     NRT_REQUIRE(!pending, NRT_ERR_INVALID, "a launch is already in flight");
     NRT_REQUIRE(elem_budget <= 0 || is_implicit(), NRT_ERR_UNSUPPORTED,
@@ -388,7 +389,7 @@ struct nrt_batch {
       // (the ticket leaves at most one neurite's workgroups waiting for others to start)
       int most = 0;
       for (const ResClass& c : res) most = std::max(most, c.maxG);
-      held = device_share(device, order.empty() || !is_implicit() ? most : INT_MAX);
+      if (!shared) held = device_share(device, order.empty() || !is_implicit() ? most : INT_MAX);
       NRT_HIP(hipEventRecord(ev0, stream));
       launch_resident(k, elem_budget, kmax, cs, ss);
       if (order.empty()) {
@@ -456,7 +457,7 @@ struct nrt_batch {
       int waiting = 0;  // workgroups of a launch with virtual grids
       for (size_t i = 0; i < order.size(); i++)
         if (vn[i] > 1) waiting = nwg;
-      if (waiting > 1 && !held) held = device_share(device, waiting);
+      if (waiting > 1 && !held && !shared) held = device_share(device, waiting);
       // (after the resident slots' launch on the same stream: workgroups that wait for
       // each other are never resident beside another such launch's)
       int64_t best = -1;
@@ -1073,8 +1074,9 @@ void batch_slot_drop(nrt_batch* b, int slot) {
 }
 
 void batch_launch(nrt_batch* b, long long k) { b->launch(k); }
-void batch_launch_budget(nrt_batch* b, long long k, long long elem_budget, long long kmax) {
-  b->launch(k, elem_budget, kmax);
+void batch_launch_budget(nrt_batch* b, long long k, long long elem_budget, long long kmax,
+                         bool shared) {
+  b->launch(k, elem_budget, kmax, shared);
 }
 void batch_finish(nrt_batch* b) { b->finish(); }
 hipStream_t batch_stream(nrt_batch* b) { return b->stream; }

@@ -3065,14 +3065,14 @@ static void resident_flip(Implicit* e, int64_t num) {
 }
 static void run_persistent(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64_t a1,
                            int32_t trace_elem, int64_t interval, double* trace_dev,
-                           hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr) {
+                           hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr, int64_t gl0 = 0) {
   Implicit* e = hnd->im;
   const auto share = device_share(hnd->device, e->nblocks);
   const bool limited = getenv("NRT_SPIN_LIMIT") != nullptr;
   const auto until = std::chrono::steady_clock::now() + std::chrono::seconds(limited ? 1 : 180);
   for (int attempt = 0;; attempt++) {
     if (t0) NRT_HIP(hipEventRecord(t0, hnd->stream));
-    launch_persistent(hnd, first, num, a0, a1, trace_elem, interval, trace_dev, 0, true);
+    launch_persistent(hnd, first, num, a0, a1, trace_elem, interval, trace_dev, gl0, true);
     if (t1) NRT_HIP(hipEventRecord(t1, hnd->stream));
     if (!e->resident) {
       if (share) NRT_HIP(hipStreamSynchronize(hnd->stream));
@@ -3301,13 +3301,38 @@ void implicit_batch_launch(int precision, int krylov, int threads, const void* w
 }
 
 // Steps first..first+num-1 enqueued on the handle's stream without waiting; the
-// trace continues a run whose phase is gl0 (steps since its last sample).
-void implicit_steps_async(nrt_handle* h, int64_t first, int64_t num, int64_t a0, int64_t a1,
+// trace continues a run whose phase is gl0 (steps since its last sample). The caller
+// holds the CUs of implicit_workgroups() (device_share) until it has waited for the
+// stream, gives them back and calls implicit_steps_end with the same arguments.
+void implicit_steps_begin(nrt_handle* h, int64_t first, int64_t num, int64_t a0, int64_t a1,
                           int32_t trace_elem, int64_t interval, int64_t gl0, double* trace_dev) {
-  launch_persistent(h, first, num, a0, a1, trace_elem, interval, trace_dev, gl0);
-  if (h->im->resident) resident_flip(h->im, num);
-  h->im->step = first + num;
+  launch_persistent(h, first, num, a0, a1, trace_elem, interval, trace_dev, gl0, true);
 }
+
+// The end of steps begun, after the stream has been waited for. A launch that gave up
+// (resident rows: its workgroups did not all start in time) is tried again here as a run
+// is; false where that fails too: the state is then the one before these steps.
+bool implicit_steps_end(nrt_handle* h, int64_t first, int64_t num, int64_t a0, int64_t a1,
+                        int32_t trace_elem, int64_t interval, int64_t gl0, double* trace_dev) {
+  Implicit* e = h->im;
+  if (e->resident) {
+    if (e->rword.p && e->rword.get()) {
+      e->rword.clear();
+      run_persistent(h, first, num, a0, a1, trace_elem, interval, trace_dev, nullptr, nullptr,
+                     gl0);
+      NRT_HIP(hipStreamSynchronize(h->stream));
+      const unsigned err = e->rerr;
+      e->rerr = 0;
+      if (err) return false;
+    } else {
+      resident_flip(e, num);
+    }
+  }
+  e->step = first + num;
+  return true;
+}
+
+int implicit_workgroups(const nrt_handle* h) { return h->im->nblocks; }
 
 // Status and inner-iteration count of a slot (its failure is reported, not cleared).
 void implicit_slot_stats_on(nrt_handle* h, hipStream_t s, int* status, int64_t* inner) {

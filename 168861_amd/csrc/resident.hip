@@ -396,7 +396,9 @@ __device__ __forceinline__ void resident_steps(const ImpDev& d, const ResDev& r,
       }
       lds_sync();
       if (*s.fail) {  // uniform: read after the barrier
-        if (tid == 0 && g == r.owner && d.st->status == NRT_OK) {
+        // (a launch from one buffer to the other has spoiled nothing: the host, which
+        // reads *d.err, tries it again)
+        if (tid == 0 && g == r.owner && r.xo == r.x && d.st->status == NRT_OK) {
           d.st->status = NRT_ERR_HIP;
           d.st->fail_step = step;
         }

@@ -20,6 +20,7 @@
 // Latency of a request = completion time - submission time (steady clock).
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <condition_variable>
 #include <cstring>
 #include <deque>
@@ -93,12 +94,14 @@ struct Result {
   std::vector<double> V, trace;
 };
 
-// A large request on a handle of its own (grid mode), stepped k at a time.
+// A large request on a handle of its own, stepped k at a time.
 struct BigRun {
   Request req;
   nrt_handle* h = nullptr;
   DBuf<double> trace;
-  int64_t done = 0;
+  int64_t done = 0, sent = 0;  // steps taken; steps in flight
+  bool failed = false;
+  int64_t left() const { return failed ? 0 : req.num_steps - done; }
   ~BigRun() {
     if (h) handle_destroy(h);
   }
@@ -303,20 +306,40 @@ struct nrt_server {
     got.clear();
   }
 
+  // CUs that the large requests' launches need at once (they follow each other on the
+  // batch stream, and the batch's launch).
+  int big_cus() const {
+    int n = 0;
+    for (const auto& b : big)
+      if (b->left() > 0) n = std::max(n, implicit_workgroups(b->h));
+    return n;
+  }
+
+  template <class F>
+  static auto big_steps(BigRun& b, F&& f) {
+    const Request& r = b.req;
+    double* tr = nullptr;
+    int64_t gl0 = 0;
+    if (r.every >= 0 && b.trace.p) {
+      tr = b.trace.p + b.done / (r.every + 1);
+      gl0 = b.done % (r.every + 1);
+    }
+    return f(b.h, b.done + 1, b.sent, r.a0, r.a1, r.trace_elem, r.every, gl0, tr);
+  }
   void launch_big(long long k) {
     for (auto& b : big) {
-      const int64_t n = std::min<int64_t>(k, b->req.num_steps - b->done);
-      if (n <= 0) continue;
-      const Request& r = b->req;
-      const int64_t every = r.every;
-      double* tr = nullptr;
-      int64_t gl0 = 0;
-      if (every >= 0 && b->trace.p) {
-        tr = b->trace.p + b->done / (every + 1);
-        gl0 = b->done % (every + 1);
-      }
-      implicit_steps_async(b->h, b->done + 1, n, r.a0, r.a1, r.trace_elem, every, gl0, tr);
-      b->done += n;
+      b->sent = std::min<int64_t>(k, b->left());
+      if (b->sent > 0) big_steps(*b, implicit_steps_begin);
+    }
+  }
+  // After the batch stream has been waited for. A request whose workgroups could not be
+  // made to run together fails; its potentials are those of its last step.
+  void finish_big() {
+    for (auto& b : big) {
+      if (b->sent <= 0) continue;
+      if (big_steps(*b, implicit_steps_end)) b->done += b->sent;
+      else b->failed = true;
+      b->sent = 0;
     }
   }
 
@@ -350,7 +373,7 @@ struct nrt_server {
     int freed = 0;
     for (auto it = big.begin(); it != big.end();) {
       BigRun& b = **it;
-      if (b.done < b.req.num_steps) {
+      if (b.left() > 0) {
         ++it;
         continue;
       }
@@ -358,14 +381,16 @@ struct nrt_server {
       if (cfg.keep_results) {
         V.resize(b.req.N());
         implicit_snapshot(b.h, V.data());
-        tr.resize(b.trace.n);
-        if (b.trace.n)
-          NRT_HIP(hipMemcpy(tr.data(), b.trace.p, sizeof(double) * b.trace.n,
+        if (b.trace.n) {
+          tr.resize(std::min<size_t>(b.trace.n, (size_t)(b.done / (b.req.every + 1))));
+          NRT_HIP(hipMemcpy(tr.data(), b.trace.p, sizeof(double) * tr.size(),
                             hipMemcpyDeviceToHost));
+        }
       }
       int status = NRT_OK;
       int64_t inner = 0;
-      implicit_slot_stats(b.h, &status, &inner);
+      if (b.failed) status = NRT_ERR_HIP;
+      else implicit_slot_stats(b.h, &status, &inner);
       finish_request(b.req, status, std::move(V), std::move(tr), b.done);
       it = big.erase(it);
       freed++;
@@ -405,19 +430,24 @@ struct nrt_server {
           stats.running = (int64_t)(running.size() + big.size() + got.size());
         }
         const double t0 = now_s();
+        double t1 = t0;
         join_ready(got);
         const long long k = cfg.steps_per_launch;
         const bool stepping = !running.empty() || !big.empty();
         if (stepping) {
-          if (opt.kind == NRT_IMPLICIT) batch_launch_budget(batch, k, k * kBudgetElems, 8 * k);
+          // the batch and the large requests' workgroups in one request for the device
+          // (asking for more while holding some could wait for one that does the same)
+          const int cus = big_cus();
+          const auto share = device_share(opt.device, running.empty() ? cus : cus > 1 ? INT_MAX : 0);
+          if (opt.kind == NRT_IMPLICIT)
+            batch_launch_budget(batch, k, k * kBudgetElems, 8 * k, share != nullptr);
           else batch_launch(batch, k);
           launch_big(k);
-        }
-        const double t1 = now_s();
-        if (stepping) {
+          t1 = now_s();
           batch_finish(batch);
           NRT_HIP(hipStreamSynchronize(batch_stream(batch)));
         }
+        finish_big();
         const double t2 = now_s();
         // The slots this launch completed are retired at once, before the next
         // launch: copies on another stream while a launch runs were found to wait
