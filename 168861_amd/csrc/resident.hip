@@ -396,12 +396,15 @@ __device__ __forceinline__ void resident_steps(const ImpDev& d, const ResDev& r,
       }
       lds_sync();
       if (*s.fail) {  // uniform: read after the barrier
-        // (a launch from one buffer to the other has spoiled nothing: the host, which
-        // reads *d.err, tries it again)
-        if (tid == 0 && g == r.owner && r.xo == r.x && d.st->status == NRT_OK) {
-          d.st->status = NRT_ERR_HIP;
+        // A launch from one buffer to the other has spoiled nothing: the host, which reads
+        // *d.err, tries it again. In place, other groups may have taken the launch's last
+        // step, so whichever gives up says that the neurite's state is lost.
+        int ok = NRT_OK;
+        if (tid == 0 && r.xo == r.x &&
+            __hip_atomic_compare_exchange_strong(&d.st->status, &ok, (int)NRT_ERR_HIP,
+                                                 __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
           d.st->fail_step = step;
-        }
         return;
       }
       for (int h = 0; h < r.top_narrow; h++) {
