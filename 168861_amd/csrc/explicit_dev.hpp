@@ -68,13 +68,6 @@ struct Explicit {
 // 8 B, 128 KiB of LDS).
 constexpr int kResMaxN = 8192;
 
-// x / c from y = 1 / c (rounded): the quotient's first estimate, its exact remainder,
-// one correction; infinite x as a division takes it.
-__device__ __forceinline__ double div_by(double x, double c, double y) {
-  const double q = x * y;
-  return __builtin_amdgcn_div_fixup(fma(fma(-c, q, x), y, q), c, x);
-}
-
 // A value that workgroups exchange: two words of 32 data bits, each with the exchange's
 // number, so that whoever polls them needs no other flag.
 typedef __attribute__((address_space(1))) unsigned long long ExWord;

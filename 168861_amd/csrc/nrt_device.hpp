@@ -101,6 +101,13 @@ __device__ __forceinline__ double rcp_newton(double x) {
   return fma(fma(-x, r, 1.0), r, r);
 }
 
+// x / c from y = 1 / c (rounded): the quotient's first estimate, its exact remainder,
+// one correction; infinite x as a division takes it.
+__device__ __forceinline__ double div_by(double x, double c, double y) {
+  const double q = x * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-c, q, x), y, q), c, x);
+}
+
 // Sum of NV values over the block (blockDim.x a multiple of 64, <= 1024); the
 // result is returned to every thread. lds must hold NV*16 doubles.
 template <int NV>

@@ -56,18 +56,25 @@ __device__ __forceinline__ void dyn_load(const ImpDev& d, const ResDev& r, int j
 // six), the diagonal and the right-hand side of the next step.
 __device__ __forceinline__ void dyn_update(DynRow& y, const ImpDev& d, int lane, bool active,
                                            double& diag, double& b) {
-  const int k = lane & 7;
+  int k = lane & 7;
+  asm volatile("" : "+v"(k));  // what depends on it is made again every step: kept, it would
+                               // cost every wave of the workgroup its registers
   const double v = y.v;
   double kdx = y.kd;
   diag = y.diag0;
   if (y.hh >= 0) {
     const bool na = k < 4;  // m and h follow the sodium shift, n the potassium shift
-    const double u = ((v + (na ? y.q.ls_Na : y.q.ls_K)) - y.q.rest) * 1000.0;
-    // k: 0 am, 1 bm, 2 ah, 3 bh, 4 an, 5 bn; exp(c0 + c1 u)
-    const double c0 = k == 0 ? 2.5 : k == 3 ? 3.0 : k == 4 ? 1.0 : 0.0;
-    const double c1 = k == 1 ? -1.0 / 18 : k == 2 ? -1.0 / 20 : k == 5 ? -1.0 / 80 : -0.1;
-    const double e = exp(fma(c1, u, c0));
-    const double num = k == 0 ? 2.5 - 0.1 * u : k == 4 ? 0.1 - 0.01 * u : 1.0;
+    const double u = div_by((v + (na ? y.q.ls_Na : y.q.ls_K)) - y.q.rest, 0.001, 1000.0);
+    // k: 0 am, 1 bm, 2 ah, 3 bh, 4 an, 5 bn; the operations of hh_rates: near 25 and 10 mV
+    // am and an are quotients of two small numbers, whose errors cancel only where both
+    // come from one rounded c0 - 0.1 u
+    const bool quot = k == 0 || k == 3 || k == 4;
+    const double c0 = k == 0 ? 2.5 : k == 3 ? 3.0 : 1.0;
+    const double c1 = k == 1 ? 18.0 : k == 2 ? 20.0 : 80.0;
+    const double y1 = k == 1 ? 1.0 / 18.0 : k == 2 ? 1.0 / 20.0 : 1.0 / 80.0;
+    const double lin = c0 - 0.1 * u;
+    const double e = exp(quot ? lin : div_by(-u, c1, y1));
+    const double num = k == 0 ? lin : k == 4 ? 0.1 - 0.01 * u : 1.0;
     const double frac = num / (k == 3 ? e + 1 : e - 1);
     const double rate = k == 1 ? 4 * e : k == 2 ? 0.07 * e : k == 5 ? 0.125 * e : frac;
     const int base = (lane & ~7) * 4;
