@@ -6,9 +6,11 @@
 #include <algorithm>
 #include <chrono>
 #include <climits>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <memory>
+#include <thread>
 #include "batch.hpp"
 
 namespace nrt {
@@ -58,7 +60,7 @@ void explicit_tree_shape(nrt_handle* h, int* groups, int* T);
 void explicit_tree_fill(nrt_handle* h, unsigned* err, long long a0, long long a1, int trace_elem,
                         long long interval, double* trace, void* out);
 void explicit_tree_work(nrt_handle* h, long long done, long long steps, void* out);
-void explicit_tree_undo(nrt_handle* h, const void* work, long long* steps);
+void explicit_tree_undo(nrt_handle* h, const void* work, long long* done, long long* steps);
 void explicit_tree_batch_launch(const void* recs, const void* work, const int2* map,
                                 unsigned* ticket, int nwg, int T, hipStream_t s);
 
@@ -326,7 +328,6 @@ struct nrt_batch {
     if (n == 0) return;
     const size_t wb = work_bytes();
     rwork_h.assign(n * wb + 4 * sizeof(unsigned), 0);  // steps, tickets
-    const size_t tick_at = n * wb;
     size_t at = 0;
     for (ResClass& c : res)
       for (int id : c.ids) {
@@ -347,6 +348,10 @@ struct nrt_batch {
         cs += w.steps * s.N;
         at++;
       }
+    enqueue_resident();
+  }
+  void enqueue_resident() {
+    const size_t tick_at = rwork_h.size() - 4 * sizeof(unsigned);
     if (rwork.n < rwork_h.size()) rwork.alloc(2 * rwork_h.size());
     NRT_HIP(hipMemcpyAsync(rwork.p, rwork_h.data(), rwork_h.size(), hipMemcpyHostToDevice, stream));
     for (int c = 0; c < 2; c++) {
@@ -380,8 +385,12 @@ struct nrt_batch {
     NRT_REQUIRE(elem_budget <= 0 || is_implicit(), NRT_ERR_UNSUPPORTED,
                 "explicit batches step in lockstep");
     if (dirty) rebuild();
-    g += k;
-    if ((order.empty() && !any_resident()) || k == 0) return;
+    if ((order.empty() && !any_resident()) || k == 0) {
+      g += k;
+      return;
+    }
+    NRT_REQUIRE(is_implicit() || order.empty() || k <= (1ll << 30), NRT_ERR_INVALID,
+                "k too large for one call");
     int64_t cs = 0, ss = 0, ccs[kClasses] = {0, 0, 0};
     pend_launches = 0;
     std::shared_ptr<void> held;  // (given back at once if the launch fails)
@@ -392,7 +401,14 @@ struct nrt_batch {
       if (!shared) held = device_share(device, order.empty() || !is_implicit() ? most : INT_MAX);
       NRT_HIP(hipEventRecord(ev0, stream));
       launch_resident(k, elem_budget, kmax, cs, ss);
+      // explicit slots take their steps together: those of the graph follow once no
+      // exchange of these has timed out
+      if (!is_implicit() && !order.empty() && most > 1) {
+        NRT_HIP(hipStreamSynchronize(stream));
+        settle_exchanges();
+      }
       if (order.empty()) {
+        g += k;
         for (ClassLaunch& c : pend_cls) c.on = false;
         NRT_HIP(hipEventRecord(ev1, stream));
         pend_cs = cs;
@@ -402,6 +418,7 @@ struct nrt_batch {
         return;
       }
     }
+    g += k;
     int th[kClasses] = {0, 0, 0};
     std::vector<int2> seg;  // wgmap range of each class
     bool merged = false;    // one launch for all classes
@@ -496,7 +513,6 @@ struct nrt_batch {
         if (pend_cls[c].on) NRT_HIP(hipStreamWaitEvent(stream, cev[c][1], 0));
       NRT_HIP(hipEventRecord(ev1, stream));
     } else {
-      NRT_REQUIRE(k <= (1ll << 30), NRT_ERR_INVALID, "k too large for one call");
       if (!gexec || graph_k != k) {
         drop_graph();
         NRT_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
@@ -568,21 +584,39 @@ struct nrt_batch {
     return seg;
   }
 
-  // Explicit slots of several workgroups: if an exchange timed out, every resident slot is
-  // where it was before the launch, and an error says so.
-  void check_exchanges() {
-    if (!rerr.p || !rerr.get()) return;
-    rerr.clear();
-    size_t at = 0;
-    for (ResClass& c : res)
-      for (int id : c.ids) {
-        long long steps = 0;
-        explicit_tree_undo(slots[id]->h, rwork_h.data() + at++ * work_bytes(), &steps);
-        slots[id]->done -= steps;
+  // Explicit slots of several workgroups, once their launch has ended: if an exchange timed
+  // out (another process holds part of the device), every resident slot goes back to where
+  // it was (it has both potentials) and the launch is tried again, for as long as a run is;
+  // then an error says so, with every slot of the batch where it was before the call.
+  void settle_exchanges() {
+    if (!rerr.p) return;
+    const auto until = std::chrono::steady_clock::now() +
+                       std::chrono::seconds(getenv("NRT_SPIN_LIMIT") ? 1 : 180);
+    for (int attempt = 0; rerr.get(); attempt++) {
+      rerr.clear();
+      const bool again = std::chrono::steady_clock::now() < until;
+      size_t at = 0;
+      for (ResClass& c : res)
+        for (int id : c.ids) {
+          uint8_t* w = rwork_h.data() + at++ * work_bytes();
+          long long done = 0, steps = 0;
+          explicit_tree_undo(slots[id]->h, w, &done, &steps);
+          if (again) explicit_tree_work(slots[id]->h, done, steps, w);
+          else slots[id]->done = done;
+        }
+      if (!again) {
+        stats.launches += pend_launches;
+        throw Error(NRT_ERR_HIP,
+                    "exchange timed out inside an explicit batch kernel (another launch held part "
+                    "of the device); the slots are where they were before this call");
       }
-    throw Error(NRT_ERR_HIP,
-                "exchange timed out inside an explicit batch kernel (another launch held part "
-                "of the device); the slots are where they were before this launch");
+      std::this_thread::sleep_for(std::chrono::microseconds(
+          100 * std::min(attempt + 1, 50) + (int)((uint32_t)((uintptr_t)this >> 6) * 2654435761u >> 22)));
+      NRT_HIP(hipEventRecord(ev0, stream));
+      enqueue_resident();
+      NRT_HIP(hipEventRecord(ev1, stream));
+      NRT_HIP(hipStreamSynchronize(stream));
+    }
   }
 
   // Waits for the launch in flight and accounts for it.
@@ -613,8 +647,8 @@ struct nrt_batch {
       stats.threads = pend_threads;
     } else {
       NRT_HIP(hipEventSynchronize(ev1));
+      settle_exchanges();
       NRT_HIP(hipEventElapsedTime(&ms, ev0, ev1));
-      check_exchanges();
     }
     stats.launches += pend_launches;
     stats.kernel_ms += ms;

@@ -517,10 +517,11 @@ void explicit_tree_work(nrt_handle* h, long long done, long long steps, void* ou
   e->cur = 1 - e->cur;
 }
 // A launch that timed out: the potentials before it are the current ones again.
-void explicit_tree_undo(nrt_handle* h, const void* work, long long* steps) {
+void explicit_tree_undo(nrt_handle* h, const void* work, long long* done, long long* steps) {
   ExTreeWork w;
   memcpy(&w, work, sizeof(w));
   h->ex->cur = w.cur;
+  *done = w.done;
   *steps = w.steps;
 }
 void explicit_tree_batch_launch(const void* recs, const void* work, const int2* map,
