@@ -44,7 +44,7 @@ namespace nrt {
 
 // krylov_block.hip
 bool krylov_block_ok(int N, bool gmres, bool mixed, int restart, int max_lds);
-void krylov_block_prepare(int N, bool gmres, int m);
+void krylov_block_prepare(int N, bool gmres, int m, int max_lds);
 void bicgstab_block_launch(ImpDev d, hipStream_t s);
 void gmres_block_launch(ImpDev d, GmresDev<double> g, hipStream_t s);
 // resident.hip
@@ -2398,7 +2398,7 @@ Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threa
                                     hnd->device));
       e->krylov_block = krylov_block_ok(N, o.krylov == NRT_GMRES, mixed, o.restart, max_lds);
       if (e->krylov_block)
-        krylov_block_prepare(N, o.krylov == NRT_GMRES, std::min(o.restart, N));
+        krylov_block_prepare(N, o.krylov == NRT_GMRES, std::min(o.restart, N), max_lds);
     }
     if (!precond && !e->krylov_block && (o.krylov == NRT_BICGSTAB || o.krylov == NRT_GMRES)) {
       // GMRES: the residual (r0), and in FP64 its Arnoldi vectors (s, t)
@@ -2556,8 +2556,9 @@ Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threa
         e->local_res = lay.total + 1024 <= (size_t)max_lds &&
                        (e->plan_h.top_n == 0 || e->plan_h.top_lds_ok);
         if (e->local_res) {
+          // (the kernel's limit, which handles of other sizes share: what any may ask for)
           NRT_HIP(hipFuncSetAttribute(kr, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)lay.total));
+                                      max_lds - 1024));
           NRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kr, kLocalBlock, lay.total));
           e->local_res = G <= cus * per_cu;
         }
@@ -2579,7 +2580,7 @@ Implicit* implicit_create(nrt_handle* hnd, const HostProblem& p, int batch_threa
             const void* kl = f64 ? (const void*)k_implicit_tree_local<double, false>
                                  : (const void*)k_implicit_tree_local<float, false>;
             NRT_HIP(hipFuncSetAttribute(kl, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)lay.top));
+                                        max_lds - 1024));
           }
         }
       }

@@ -657,9 +657,10 @@ static size_t kg_lds(int N, int m) {
 // that the grid kernel gives to one workgroup; with 8 rows for each of 512 threads,
 // 4,000 rows took 5.9 us an iteration against 33, but in another order of sums than the
 // grid of two.
+constexpr int kKbStaticLds = 4096;  // at most, beside the dynamic LDS
 bool krylov_block_ok(int N, bool gmres, bool mixed, int restart, int max_lds) {
   if (N > (gmres ? kKgMaxN : kKbMaxN) || mixed) return false;
-  return (gmres ? kg_lds(N, std::min(restart, N)) : kb_lds(N)) + 4096 <= (size_t)max_lds;
+  return (gmres ? kg_lds(N, std::min(restart, N)) : kb_lds(N)) + kKbStaticLds <= (size_t)max_lds;
 }
 
 struct KbShape {
@@ -686,11 +687,13 @@ static KbShape gmres_shape(int N, int m) {
   return KbShape{k, half, kg_lds(N, m)};
 }
 
-// Once per handle: the kernel may use the LDS that its launches ask for.
-void krylov_block_prepare(int N, bool gmres, int m) {
+// Once per handle: the kernel may use the LDS that its launches ask for (as much as any
+// handle asks for: the limit is the kernel's, and handles of other sizes share it).
+void krylov_block_prepare(int N, bool gmres, int m, int max_lds) {
   const KbShape q = gmres ? gmres_shape(N, m) : bicgstab_shape(N);
   if (q.lds > 48 * 1024)
-    NRT_HIP(hipFuncSetAttribute(q.k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)q.lds));
+    NRT_HIP(hipFuncSetAttribute(q.k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                max_lds - kKbStaticLds));
 }
 
 void bicgstab_block_launch(ImpDev d, hipStream_t s) {
