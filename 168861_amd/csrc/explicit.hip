@@ -277,6 +277,7 @@ Explicit* explicit_create(nrt_handle* hnd, const HostProblem& p, bool in_batch) 
   const int N = p.N, H = p.H;
   auto* e = new Explicit;
   try {
+    ExPlan ahead = tree_plan(hnd, p, in_batch);
     e->N = N;
     e->H = H;
     e->dT = p.dT;
@@ -386,7 +387,7 @@ Explicit* explicit_create(nrt_handle* hnd, const HostProblem& p, bool in_batch) 
     e->hdx.upload(hdx, s);
     cable_prepare(hnd, e, p, in_batch);
     ExPlanHost plan;
-    if (e->cable_groups == 0) tree_prepare(hnd, e, p, in_batch, plan);
+    if (e->cable_groups == 0) tree_prepare(hnd, e, p, plan = ahead.get());
     NRT_HIP(hipStreamSynchronize(s));
   } catch (...) {
     delete e;

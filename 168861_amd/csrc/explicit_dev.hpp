@@ -2,6 +2,7 @@
 // small neurites in one workgroup, batches; explicit_cable.hip: unbranched neurites).
 #pragma once
 #include <functional>
+#include <future>
 #include "explicit_tree.hpp"
 #include "nrt_device.hpp"
 #include "nrt_internal.hpp"
@@ -130,8 +131,10 @@ bool cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t
                int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0, hipEvent_t t1);
 
 // explicit_tree.hip
-void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_batch,
-                  ExPlanHost& P);
+// The plan (G = 0: none), begun; it reads p until it has been got.
+using ExPlan = std::future<ExPlanHost>;
+ExPlan tree_plan(nrt_handle* hnd, const HostProblem& p, bool in_batch);
+void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, const ExPlanHost& P);
 bool tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
               int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0, hipEvent_t t1);
 

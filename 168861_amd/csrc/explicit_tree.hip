@@ -20,6 +20,7 @@
 #include <climits>
 #include <cstdlib>
 #include <cstring>
+#include <system_error>
 #include "explicit_dev.hpp"
 
 namespace nrt {
@@ -429,31 +430,47 @@ int tree_capacity(int device, int T) {
 }
 }  // namespace
 
-// (P: the plan is uploaded from it until the stream is waited for)
-void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_batch,
-                  ExPlanHost& P) {
-  // (a run of an unbranched neurite is the cable kernel's or specified as a launch a step)
-  bool branching = in_batch;
-  for (int j = 1; j < p.N - 1 && !branching; j++) branching = p.branching[j] != 0;
-  if (!branching) return;
-  std::string why;
-  bool fits = false;
+constexpr int kExPlanAlone = 16384;  // elements
+
+// The plan, of a large handle on a thread of its own beside the rest of the creation: a
+// handle that is only stepped has no use for it. Creation in ms without a plan, with it made
+// in line, and so: 902,037 elements 19.1, 26.9, 20.1; 200,000 2.0, 3.4, 2.5; 30,000 0.39,
+// 0.54, 0.46; 17,000 0.29, 0.37, 0.36 (below kExPlanAlone in line: the thread costs as much).
+ExPlan tree_plan(nrt_handle* hnd, const HostProblem& p, bool in_batch) {
+  // (a run of an unbranched neurite is the cable kernel's or specified as a launch a step;
+  // one or two steps are no run of this form)
   const int cap = tree_capacity(hnd->device, kExT);
-  const auto plan = [&](int T, int most) {
-    // (strands of some 50 elements and halos: 4 to 6% more units than N / kExC)
-    if (p.N / kExC * 1.03 > (double)most * T) return;
-    for (int every : {kExEvery, kExEveryDense})
-      if (!fits && build_explicit_plan(p, T, every, P, why)) fits = P.G <= most;
+  const auto make = [&p, in_batch, cap] {
+    ExPlanHost P;
+    bool branching = in_batch, fits = false;
+    for (int j = 1; j < p.N - 1 && !branching; j++) branching = p.branching[j] != 0;
+    std::string why;
+    const auto plan = [&](int T, int most) {
+      // (strands of some 50 elements and halos: 4 to 6% more units than N / kExC)
+      if (!branching || p.N / kExC * 1.03 > (double)most * T) return;
+      for (int every : {kExEvery, kExEveryDense})
+        if (!fits && build_explicit_plan(p, T, every, P, why)) fits = P.G <= most;
+    };
+    // (larger groups where there are not CUs enough: seven or eight waves of units)
+    plan(kExTBatch, cap);
+    if (!in_batch && !fits) plan(kExTLarge, cap);
+    if (!in_batch && !fits) plan(kExT, cap);
+    if (!fits) P = ExPlanHost();
+    return P;
   };
-  // (larger groups where there are not CUs enough: seven or eight waves of units)
-  plan(kExTBatch, cap);
-  if (!in_batch && !fits) plan(kExTLarge, cap);
-  if (!in_batch && !fits) plan(kExT, cap);
-  if (!fits) return;
-  e->tree_groups = P.G;
-  e->tree_T = P.T;
-  e->tree_slots = P.slots;
-  e->tree_every = P.every;
+  if (!in_batch && p.N >= kExPlanAlone) {
+    try {
+      return std::async(std::launch::async, make);
+    } catch (const std::system_error&) {  // (no thread to be had)
+    }
+  }
+  return std::async(std::launch::deferred, make);
+}
+
+// The plan's device state; leaves the solver without the form where the plan refuses. (P:
+// uploaded from until the stream is waited for)
+void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, const ExPlanHost& P) {
+  if (P.G == 0) return;
   e->tunit.upload(P.unit, hnd->stream);
   e->tdyn.upload(P.dyn, hnd->stream);
   e->m2.alloc(p.H);
@@ -464,6 +481,10 @@ void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_ba
     e->ll.alloc((size_t)2 * P.slots * kExSlotVals * 2);
     NRT_HIP(hipMemsetAsync(e->ll.p, 0, sizeof(unsigned long long) * e->ll.n, hnd->stream));
   }
+  e->tree_groups = P.G;
+  e->tree_T = P.T;
+  e->tree_slots = P.slots;
+  e->tree_every = P.every;
 }
 
 static ExTreeDev tree_dev(Explicit* e, int from, unsigned* err, long long a0, long long a1,
