@@ -430,7 +430,20 @@ int tree_capacity(int device, int T) {
 }
 }  // namespace
 
+// Device memory of the plan beyond what a batch's admission reckons with per element is
+// only taken while this much stays free for other slots.
+constexpr int64_t kExPlanBytesPerElem = 12;
+constexpr int64_t kExPlanReserve = 512ll << 20;
 constexpr int kExPlanAlone = 16384;  // elements
+
+static bool tree_room(int device, const ExPlanHost& P) {
+  const int64_t bytes = (int64_t)(P.unit.size() * sizeof(ExUnit) + P.dyn.size() * sizeof(ExDynUnit)) +
+                        (int64_t)P.slots * 2 * kExSlotVals * 2 * 8;
+  if (bytes <= kExPlanBytesPerElem * P.N) return true;
+  size_t free_b = 0, total_b = 0;
+  NRT_HIP(hipMemGetInfo(&free_b, &total_b));
+  return (int64_t)free_b + pool_cached_bytes(device) >= bytes + kExPlanReserve;
+}
 
 // The plan, of a large handle on a thread of its own beside the rest of the creation: a
 // handle that is only stepped has no use for it. Creation in ms without a plan, with it made
@@ -467,20 +480,28 @@ ExPlan tree_plan(nrt_handle* hnd, const HostProblem& p, bool in_batch) {
   return std::async(std::launch::deferred, make);
 }
 
-// The plan's device state; leaves the solver without the form where the plan refuses. (P:
-// uploaded from until the stream is waited for)
+// The plan's device state; leaves the solver without the form where the plan refuses or the
+// memory is not there. (P: uploaded from until the stream is waited for)
 void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, const ExPlanHost& P) {
-  if (P.G == 0) return;
-  e->tunit.upload(P.unit, hnd->stream);
-  e->tdyn.upload(P.dyn, hnd->stream);
-  e->m2.alloc(p.H);
-  e->h2.alloc(p.H);
-  e->n2.alloc(p.H);
-  e->err.take();
-  if (P.slots > 0) {
-    e->ll.alloc((size_t)2 * P.slots * kExSlotVals * 2);
-    NRT_HIP(hipMemsetAsync(e->ll.p, 0, sizeof(unsigned long long) * e->ll.n, hnd->stream));
+  if (P.G == 0 || !tree_room(hnd->device, P)) return;
+  try {
+    e->tunit.upload(P.unit, hnd->stream);
+    e->tdyn.upload(P.dyn, hnd->stream);
+    e->m2.alloc(p.H);
+    e->h2.alloc(p.H);
+    e->n2.alloc(p.H);
+    if (P.slots > 0) e->ll.alloc((size_t)2 * P.slots * kExSlotVals * 2);
+  } catch (const Error& err) {
+    if (err.status != NRT_ERR_NOMEM) throw;
+    NRT_HIP(hipStreamSynchronize(hnd->stream));
+    e->tunit.release();
+    e->tdyn.release();
+    for (DBuf<double>* b : {&e->m2, &e->h2, &e->n2}) b->release();
+    return;
   }
+  e->err.take();
+  if (P.slots > 0)
+    NRT_HIP(hipMemsetAsync(e->ll.p, 0, sizeof(unsigned long long) * e->ll.n, hnd->stream));
   e->tree_groups = P.G;
   e->tree_T = P.T;
   e->tree_slots = P.slots;
