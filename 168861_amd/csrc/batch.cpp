@@ -62,7 +62,7 @@ void explicit_tree_fill(nrt_handle* h, unsigned* err, long long a0, long long a1
 void explicit_tree_work(nrt_handle* h, long long done, long long steps, void* out);
 void explicit_tree_undo(nrt_handle* h, const void* work, long long* done, long long* steps);
 void explicit_tree_batch_launch(const void* recs, const void* work, const int2* map,
-                                unsigned* ticket, int nwg, int T, hipStream_t s);
+                                unsigned* ticket, int nwg, int T, bool one, hipStream_t s);
 
 namespace {
 // Workgroup sizes the autotuner tries, in this order, for each size class of slots.
@@ -143,6 +143,7 @@ struct nrt_batch {
   DBuf<int2> rmap;
   std::vector<uint8_t> rwork_h;
   HostWord rerr;  // explicit: an exchange timed out
+  bool rone = false;  // explicit: the launch takes one step of every slot
   DBuf<uint8_t> table;
   DBuf<int2> blk;
   int nblk = 0;
@@ -328,6 +329,7 @@ struct nrt_batch {
     if (n == 0) return;
     const size_t wb = work_bytes();
     rwork_h.assign(n * wb + 4 * sizeof(unsigned), 0);  // steps, tickets
+    rone = k == 1;
     size_t at = 0;
     for (ResClass& c : res)
       for (int id : c.ids) {
@@ -362,7 +364,7 @@ struct nrt_batch {
         resident_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, res[c].lds,
                               stream);
       else
-        explicit_tree_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, stream);
+        explicit_tree_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, rone, stream);
       pend_launches++;
     }
   }
