@@ -19,7 +19,7 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
     return false;
   };
   if (N < 4 || p.T < 1 || p.terminals[0] != 0) return no("first terminal");
-  std::vector<uint8_t> mark(N + 1, 0);  // 1: sealed end, 2: HH element
+  std::vector<uint8_t> mark(N + 8, 0);  // 1: sealed end, 2: HH element, 4: stimulus
   struct Bit {
     const uint8_t* m;
     uint8_t b;
@@ -41,13 +41,30 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
     return (int)(std::find(p.hh_elem.begin(), p.hh_elem.end(), e) - p.hh_elem.begin());
   };
   if (p.mother[1] != 0) return no("element 1");
+  // amid[j]: a passive, unbranched element after its mother and before its only daughter, by
+  // its own entries (eight at a time below: most elements are amid a strand)
+  std::vector<uint8_t> amid(N + 8, 0);
+  {
+    const int32_t *mo = p.mother.data(), *dr = p.dr.data();
+    const uint8_t *br = p.branching.data(), *mk = mark.data();
+    uint8_t* __restrict__ to = amid.data();
+    for (int j = 1; j < N; j++) {
+      const unsigned off = ((unsigned)mo[j] ^ (unsigned)(j - 1)) |
+                           ((unsigned)dr[j] ^ (unsigned)(j + 1)) | br[j] | mk[j];
+      to[j] = off == 0 ? 1 : 0;
+    }
+  }
+  const auto all_amid = [&](int j) {  // of j .. j + 7
+    uint64_t w;
+    std::memcpy(&w, amid.data() + j, 8);
+    return w == 0x0101010101010101ull;
+  };
   // every computed element: its daughters name it as their mother, and the other way
   auto daughter = [&](int j, int d) { return d >= 1 && d < N && p.mother[d] == j; };
   for (int j = 1; j < N; j++) {
+    while (all_amid(j - 1)) j += 6;
+    if (amid[j - 1] & amid[j] & amid[j + 1]) continue;  // (all of the below)
     const int m = p.mother[j];
-    if (j >= 2 && !(mark[j - 1] | mark[j] | mark[j + 1]) && m == j - 1 && p.dr[m] == j &&
-        !p.branching[j] && p.dr[j] == j + 1 && j + 1 < N && p.mother[j + 1] == j)
-      continue;  // (an element amid a strand: all of the below)
     if (term[j]) {
       // a sealed end: the next element after a passive, unbranched source
       if (m != j - 1 || m < 1 || term[m] || hh[m] || p.branching[m] || p.dr[m] != j)
@@ -66,6 +83,11 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
       return no("sealed end of an HH element");
     }
   }
+  {
+    const double* in = p.input.data();
+    uint8_t* __restrict__ to = mark.data();
+    for (int j = 1; j < N; j++) to[j] |= in[j] != 0.0 ? 4 : 0;
+  }
   // ---- nodes in element order: units (chains cut from their ends) and HH elements
   struct Node {
     int32_t first, n, last, dyn;  // dyn -1: a unit
@@ -82,6 +104,7 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
       continue;
     }
     int e = j;  // last element of the chain that starts at j
+    while (all_amid(e)) e += 7;
     while (e + 1 < N && !term[e] && !hh[e + 1] && p.mother[e + 1] == e && p.dr[e] == e + 1 &&
            !p.branching[e])
       e++;
@@ -174,15 +197,18 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
     const auto& mem = members[g];
     // units with unused places side by side, then other ends of chains: fewer waves do
     // what only these need
-    int nu = 0, nd = 0;
-    for (int kind = 0; kind < 3; kind++)
-      for (int w : mem) {
-        const Node& q = node[w];
-        const int is = q.n < C ? 0 : (term[q.last] || q.left >= 0 ? 1 : 2);
-        if (q.dyn >= 0 ? kind != 0 : is != kind) continue;
-        in[w] = g;
-        at[w] = q.dyn < 0 ? nu++ : nd++;
-      }
+    int next[4] = {0, 0, 0, 0};  // of the kinds: 0 HH elements, 1 .. 3 units
+    const auto kind = [&](const Node& q) {
+      return q.dyn >= 0 ? 0 : q.n < C ? 1 : term[q.last] || q.left >= 0 ? 2 : 3;
+    };
+    for (int w : mem) next[kind(node[w])]++;
+    next[3] = next[1] + next[2];
+    next[2] = next[1];
+    next[0] = next[1] = 0;
+    for (int w : mem) {
+      in[w] = g;
+      at[w] = next[kind(node[w])]++;
+    }
     auto head = [&](int w) {
       if (w < 0 || in[w] != g) return (uint16_t)kExMissing;
       return (uint16_t)(node[w].dyn < 0 ? at[w] : 2 * kExT + at[w]);
@@ -198,7 +224,9 @@ bool build_explicit_plan(const HostProblem& p, int T, int every, ExPlanHost& P, 
                     (term[q.last] ? kExUTerm : 0) | (owner[w] != g ? kExUHalo : 0);
       const int er = q.right >= 0 ? p.dr[q.last] : q.last, el = q.left >= 0 ? p.dl[q.last] : q.last;
       double input = 0;
-      for (int k = 0; k < q.n; k++) {
+      uint64_t marks;  // (of the unit's elements, and perhaps some after them)
+      std::memcpy(&marks, mark.data() + q.first, 8);
+      for (int k = 0; k < q.n && (marks & 0x0404040404040404ull); k++) {
         const int j = q.first + k;
         if (term[j] || p.input[j] == 0.0) continue;
         if (fl & kExUInput) return no("two stimuli in a unit");

@@ -469,10 +469,10 @@ static bool tree_room(int device, const ExPlanHost& P) {
   return (int64_t)free_b + pool_cached_bytes(device) >= bytes + kExPlanReserve;
 }
 
-// The plan, of a large handle on a thread of its own beside the rest of the creation: a
+// The plan, of a large neurite on a thread of its own beside the rest of the creation: a
 // handle that is only stepped has no use for it. Creation in ms without a plan, with it made
-// in line, and so: 902,037 elements 19.1, 26.9, 20.1; 200,000 2.0, 3.4, 2.5; 30,000 0.39,
-// 0.54, 0.46; 17,000 0.29, 0.37, 0.36 (below kExPlanAlone in line: the thread costs as much).
+// in line, and so: 902,037 elements 19.1, 26.9, 20.0; 200,000 2.0, 3.4, 2.2; 30,000 0.39,
+// 0.54, 0.46; 17,000 0.29, 0.37, 0.34 (below kExPlanAlone in line: the thread costs as much).
 ExPlan tree_plan(nrt_handle* hnd, const HostProblem& p, bool in_batch) {
   // (a run of an unbranched neurite is the cable kernel's or specified as a launch a step;
   // one or two steps are no run of this form)
@@ -495,7 +495,7 @@ ExPlan tree_plan(nrt_handle* hnd, const HostProblem& p, bool in_batch) {
     if (!fits) P = ExPlanHost();
     return P;
   };
-  if (!in_batch && p.N >= kExPlanAlone) {
+  if (p.N >= kExPlanAlone) {
     try {
       return std::async(std::launch::async, make);
     } catch (const std::system_error&) {  // (no thread to be had)
