@@ -436,14 +436,14 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
   NRT_HIP(hipEventCreate(&t1));
   NRT_HIP(hipEventRecord(t0, hnd->stream));
   int64_t k = 0;
-  int64_t launches = num;
   double* const trace = tracing && trace_out ? e->trace.p : nullptr;
   const int32_t probe = tracing ? trace_elem : 0;
-  const bool exchanging = cable_run(hnd, e, first, num, a0, a1, probe, interval, trace, t0, t1) ||
-                          tree_run(hnd, e, first, num, a0, a1, probe, interval, trace, t0, t1);
+  int64_t launches = cable_run(hnd, e, first, num, a0, a1, probe, interval, trace, t0, t1);
+  if (launches == 0)
+    launches = tree_run(hnd, e, first, num, a0, a1, probe, interval, trace, t0, t1);
+  const bool exchanging = launches > 0;
   if (exchanging) {
     k = max_samples;
-    launches = 1;
   } else if (e->N <= kResMaxN) {
     launches = 1;
     // one launch for the whole run; the result lands in the other buffer, which
@@ -464,6 +464,7 @@ void explicit_run(nrt_handle* hnd, int64_t first, int64_t num, int64_t a0, int64
     e->cur = 1 - e->cur;
     k = max_samples;
   } else {
+    launches = num;
     int64_t gl = 0;
     for (int64_t i = first; i < first + num; i++) {
       const bool active = i >= a0 && i <= a1;

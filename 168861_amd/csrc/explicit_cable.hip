@@ -267,7 +267,7 @@ void run_exchanging(nrt_handle* hnd, Explicit* e, int G,
   const auto share = device_share(hnd->device, G > 1 ? G : 0);
   const auto until = std::chrono::steady_clock::now() + std::chrono::seconds(sl ? 1 : 180);
   for (int attempt = 0;; attempt++) {
-    NRT_HIP(hipEventRecord(t0, hnd->stream));
+    if (t0) NRT_HIP(hipEventRecord(t0, hnd->stream));
     launch(std::min(limit, 20000ull), limit);
     NRT_HIP(hipGetLastError());
     NRT_HIP(hipEventRecord(t1, hnd->stream));
@@ -290,14 +290,14 @@ void run_exchanging(nrt_handle* hnd, Explicit* e, int G,
   std::swap(e->n.p, e->n2.p);
 }
 
-bool cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
-               int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
-               hipEvent_t t1) {
+int64_t cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
+                  int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
+                  hipEvent_t t1) {
   // One step of a short neurite, or two of a very short one, are done by one workgroup
   // before this launch has set up its registers (runs of 1 / 2 / 4 steps there and here, us,
   // with the launch and the wait: 402 elements 19 / 22 / 30 and 24 / 24 / 26, 1,002
   // 21 / 26 / 36 and 24 / 25 / 27, 5,000 35 / 53 / 89 and 25 / 25 / 27).
-  if (e->cable_groups == 0 || (num <= 2 && num * e->N <= 2048)) return false;
+  if (e->cable_groups == 0 || (num <= 2 && num * e->N <= 2048)) return 0;
   const int G = e->cable_groups;
   run_exchanging(
       hnd, e, G,
@@ -311,7 +311,7 @@ bool cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t
         hipLaunchKernelGGL(k_explicit_cable, dim3(G), dim3(kCabBlock), 0, hnd->stream, q);
       },
       t0, t1);
-  return true;
+  return 1;
 }
 
 }  // namespace nrt

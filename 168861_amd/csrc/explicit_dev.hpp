@@ -126,16 +126,18 @@ void run_exchanging(nrt_handle* hnd, Explicit* e, int G,
                     const std::function<void(unsigned long long, unsigned long long)>& launch,
                     hipEvent_t t0, hipEvent_t t1);
 void cable_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, bool in_batch);
-// A run by the cable kernel, waited for; false where it does not apply.
-bool cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
-               int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0, hipEvent_t t1);
+// A run by the cable kernel, waited for; its launches (0: the kernel does not apply).
+int64_t cable_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
+                  int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
+                  hipEvent_t t1);
 
 // explicit_tree.hip
 // The plan (G = 0: none), begun; it reads p until it has been got.
 using ExPlan = std::future<ExPlanHost>;
 ExPlan tree_plan(nrt_handle* hnd, const HostProblem& p, bool in_batch);
 void tree_prepare(nrt_handle* hnd, Explicit* e, const HostProblem& p, const ExPlanHost& P);
-bool tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
-              int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0, hipEvent_t t1);
+int64_t tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
+                 int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
+                 hipEvent_t t1);
 
 }  // namespace nrt

@@ -539,24 +539,41 @@ static ExTreeDev tree_dev(Explicit* e, int from, unsigned* err, long long a0, lo
           e->m2.p, e->h2.p, e->n2.p, e->dt_ms, e->ll.p, err, a0, a1, interval, trace_elem};
 }
 
-bool tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
-              int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0, hipEvent_t t1) {
+int64_t tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
+                 int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
+                 hipEvent_t t1) {
   // One or two steps go over memory, as fast as the registers are filled and emptied (run
   // of 1 / 2 / 4 steps there and here, us, with the launch and the wait: 700 elements 18 / 20
   // / 25 and 23 / 24 / 25; 30,000 18 / 22 / 30 and 24 / 24 / 25; 902,037 23 / 33 / 53 and
   // 30 / 32 / 33).
-  if (e->tree_groups == 0 || num <= 2) return false;
-  run_exchanging(
-      hnd, e, e->tree_groups,
-      [&](unsigned long long first_limit, unsigned long long limit) {
-        const ExTreeDev d = tree_dev(e, e->cur, e->err.p, a0, a1, interval, trace_elem);
-        ExTreeRun q{0, (long long)first, (long long)num, 0, trace, e->tag, first_limit, limit};
-        e->tag += (unsigned)(num / e->tree_every + 2);
-        hipLaunchKernelGGL(k_explicit_tree, dim3(e->tree_groups), dim3(e->tree_T + kWave), 0,
-                           hnd->stream, d, q);
-      },
-      t0, t1);
-  return true;
+  if (e->tree_groups == 0 || num <= 2) return 0;
+  // (pieces: see run_persistent in implicit.hip; 8,192 steps of 902,037 elements 12 ms)
+  constexpr int64_t kShareSteps = 8192;
+  constexpr int kShareCus = 64;
+  const int64_t most = e->tree_groups > kShareCus ? kShareSteps : num;
+  const int64_t per = interval >= 0 ? interval + 1 : 1;
+  int64_t done = 0, launches = 0;
+  for (; done < num; launches++) {
+    const int64_t n = std::min(most, num - done);
+    try {
+      run_exchanging(
+          hnd, e, e->tree_groups,
+          [&](unsigned long long first_limit, unsigned long long limit) {
+            const ExTreeDev d = tree_dev(e, e->cur, e->err.p, a0, a1, interval, trace_elem);
+            ExTreeRun q{0, (long long)(first + done), (long long)n, done % per,
+                        trace ? trace + done / per : nullptr, e->tag, first_limit, limit};
+            e->tag += (unsigned)(n / e->tree_every + 2);
+            hipLaunchKernelGGL(k_explicit_tree, dim3(e->tree_groups), dim3(e->tree_T + kWave), 0,
+                               hnd->stream, d, q);
+          },
+          done == 0 ? t0 : nullptr, t1);
+    } catch (...) {
+      hnd->stats.steps += done;  // (as the statistics of the implicit forms count them)
+      throw;
+    }
+    done += n;
+  }
+  return launches;
 }
 
 // ---- slots of a batch (batch.cpp): their gates stay where they are and the work names
