@@ -610,7 +610,7 @@ struct nrt_batch {
         stats.launches += pend_launches;
         throw Error(NRT_ERR_HIP,
                     "exchange timed out inside an explicit batch kernel (another launch held part "
-                    "of the device); the slots are where they were before this call");
+                    "of the device); the slots are where they were before this launch");
       }
       std::this_thread::sleep_for(std::chrono::microseconds(
           100 * std::min(attempt + 1, 50) + (int)((uint32_t)((uintptr_t)this >> 6) * 2654435761u >> 22)));
@@ -663,9 +663,36 @@ struct nrt_batch {
         if (slots[id] && slots[id]->left() <= 0) dirty = true;
   }
 
+  // Explicit slots in registers: a call of very many steps is several launches of about
+  // 20 ms each (0.6 us a step at least, 5.5e5 elements a us), between which work of other
+  // threads gets its turn, as between the launches of single steps (30,000 steps of 2,048
+  // trees in one launch kept 20 steps of a large tree waiting for 162 ms; 15 so).
+  long long steps_per_launch(long long k) {
+    if (pending) return k;
+    if (dirty) rebuild();
+    if (is_implicit() || !order.empty() || !any_resident()) return k;
+    long long elems = 0;
+    for (const ResClass& c : res)
+      for (int id : c.ids) elems += slots[id]->N;
+    const long long n = std::max(256ll, (long long)(20000 / std::max(0.6, (double)elems / 5.5e5)));
+    return k > n + n / 2 ? n : k;
+  }
+
   void step(long long k) {
-    launch(k);
-    finish();
+    const long long most = steps_per_launch(k);
+    long long done = 0;
+    do {
+      const long long n = std::min(most, k - done);
+      try {
+        launch(n);
+        finish();
+      } catch (const Error& e) {
+        if (done == 0) throw;
+        throw Error(e.status, std::string(e.what()) + " (after " + std::to_string(done) +
+                                  " of the call's steps)");
+      }
+      done += n;
+    } while (done < k);
   }
 };
 

@@ -37,6 +37,21 @@ def test_pieces_are_one_run(form, steps, nrt):
         assert np.array_equal(s.snapshot(), one.snapshot())
 
 
+def test_batch_pieces_are_one_call(nrt):
+    """(a launch: 33,333 steps of so few elements)"""
+    p, steps = _tree(nrt, 4, "explicit"), 60000
+    with nrt.Solver(p, **FORMS["explicit"]) as s, nrt.Batch(**FORMS["explicit"]) as b:
+        tr = s.run(1, steps, 5, 40000, trace_elem=1, interval=6)
+        slots = [b.add(p, n, 5, 40000, 1, 6) for n in (steps, 35000, steps + 10)]
+        b.step(steps)
+        assert b.stats()["launches"] == 2
+        for i, n in zip(slots, (steps, 35000, steps)):
+            assert b.info(i)["steps_done"] == n
+            assert np.array_equal(b.trace(i), tr[:n // 7])
+        for i in (slots[0], slots[2]):
+            assert np.array_equal(b.snapshot(i), s.snapshot())
+
+
 def test_a_small_run_beside_a_long_one(nrt):
     large, small = _tree(nrt, 14, "direct"), _tree(nrt, 6, "direct")
     with nrt.Solver(large, **FORMS["direct"]) as a, nrt.Solver(small, **FORMS["direct"]) as b:
