@@ -128,8 +128,8 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
     // (an unused place reads what lies before the unit, or, at the arrays' beginning, the
     // unit's first element: no load waits for another)
     const int at = u.first - f;
-    const bool works = on && !(ONE && halo);
-    if (ONE && !works && at >= 0) {
+    const bool shows = ONE && halo;
+    if (shows && at >= 0) {
       ex_load8(Vin + at, V);
     } else if (on && at >= 0) {
       ex_load8(Vin + at, V);
@@ -152,13 +152,14 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
     for (int k = 0; k < C; k++) {
       const bool used = k >= f;
       V[k] = used ? V[k] : 0.0;
-      a[k] = used && works ? a[k] : 0.0;
-      r[k] = used && works ? r[k] : 1.0;
-      w[k] = used && works ? w[k] : 0.0;
-      kd[k] = used && works ? kd[k] : 0.0;
+      a[k] = used && !shows ? a[k] : 0.0;
+      r[k] = used && !shows ? r[k] : 1.0;
+      w[k] = used && !shows ? w[k] : 0.0;
+      kd[k] = used && !shows ? kd[k] : 0.0;
       y[k] = 1 / r[k];
     }
-    const double rR = works ? rdx[u.el_right] : 1.0, rL = works ? rdx[u.el_left] : 1.0;
+    const double rR = on && !shows ? rdx[u.el_right] : 1.0,
+                 rL = on && !shows ? rdx[u.el_left] : 1.0;
     const double yR = 1 / rR, yL = 1 / rL;
     double v0 = ghost ? Vin[0] : 0.0;
     const int up = on ? u.up : kExMissing, right = on && !term ? u.right : kExMissing;
