@@ -52,6 +52,11 @@ void explicit_batch_steps(const void* slots, const int2* blk, int nblk, int nslo
 const double* explicit_slot_v(nrt_handle* h, long long done);
 int64_t explicit_device_bytes(const Explicit* e);
 int explicit_batch_block_elems();
+size_t explicit_one_bytes();
+void explicit_one_fill(nrt_handle* h, long long num_steps, long long a0, long long a1,
+                       int trace_elem, long long interval, double* trace, void* out);
+void explicit_one_launch(const void* slots, const void* work, const int2* blk, int nblk,
+                         int nslots, int i, bool probes, hipStream_t s);
 // explicit_tree.hip
 bool explicit_tree_slot(const nrt_handle* h);
 size_t explicit_tree_rec_bytes();
@@ -62,7 +67,7 @@ void explicit_tree_fill(nrt_handle* h, unsigned* err, long long a0, long long a1
 void explicit_tree_work(nrt_handle* h, long long done, long long steps, void* out);
 void explicit_tree_undo(nrt_handle* h, const void* work, long long* done, long long* steps);
 void explicit_tree_batch_launch(const void* recs, const void* work, const int2* map,
-                                unsigned* ticket, int nwg, int T, bool one, hipStream_t s);
+                                unsigned* ticket, int nwg, int T, hipStream_t s);
 
 namespace {
 // Workgroup sizes the autotuner tries, in this order, for each size class of slots.
@@ -143,7 +148,11 @@ struct nrt_batch {
   DBuf<int2> rmap;
   std::vector<uint8_t> rwork_h;
   HostWord rerr;  // explicit: an exchange timed out
-  bool rone = false;  // explicit: the launch takes one step of every slot
+  // explicit: calls of one step go over memory (records and blocks, made by the first of
+  // them); those that follow each other use the first one's work, osteps later
+  DBuf<uint8_t> otable;
+  DBuf<int2> oblk;
+  int noblk = 0, osteps = -1;
   DBuf<uint8_t> table;
   DBuf<int2> blk;
   int nblk = 0;
@@ -258,6 +267,8 @@ struct nrt_batch {
   // while they fill the device (as size classes do); else all share one.
   void rebuild_resident() {
     for (ResClass& c : res) c = ResClass();
+    noblk = 0;
+    osteps = -1;
     std::vector<int> rest;
     for (int id : order) {
       if (!row_resident(id)) {
@@ -329,7 +340,6 @@ struct nrt_batch {
     if (n == 0) return;
     const size_t wb = work_bytes();
     rwork_h.assign(n * wb + 4 * sizeof(unsigned), 0);  // steps, tickets
-    rone = k == 1;
     size_t at = 0;
     for (ResClass& c : res)
       for (int id : c.ids) {
@@ -350,12 +360,54 @@ struct nrt_batch {
         cs += w.steps * s.N;
         at++;
       }
-    enqueue_resident();
+    if (!is_implicit() && k == 1) enqueue_one();
+    else enqueue_resident();
+  }
+  void upload_work() {
+    if (rwork.n < rwork_h.size()) rwork.alloc(2 * rwork_h.size());
+    NRT_HIP(hipMemcpyAsync(rwork.p, rwork_h.data(), rwork_h.size(), hipMemcpyHostToDevice, stream));
+  }
+  // One step of the explicit resident slots, over memory.
+  void enqueue_one() {
+    int n = 0;
+    bool probes = false;
+    for (ResClass& c : res)
+      for (int id : c.ids) {
+        const Slot& s = *slots[id];
+        probes = probes || (s.interval >= 0 && s.trace.p && s.done % (s.interval + 1) == 0);
+        n++;
+      }
+    if (noblk == 0) {
+      const size_t ob = explicit_one_bytes();
+      std::vector<uint8_t> host(ob * n);
+      std::vector<int2> bl;
+      int at = 0;
+      for (ResClass& c : res)
+        for (int id : c.ids) {
+          Slot& s = *slots[id];
+          explicit_one_fill(s.h, s.num_steps, s.a0, s.a1, s.trace_elem, s.interval, s.trace.p,
+                            host.data() + ob * at);
+          for (int e0 = 0; e0 < s.N; e0 += 256) bl.push_back(make_int2(at, e0));
+          at++;
+        }
+      otable.upload(host, stream);
+      oblk.upload(bl, stream);
+      NRT_HIP(hipStreamSynchronize(stream));
+      noblk = (int)bl.size();
+    }
+    if (osteps < 0 || osteps == INT_MAX) {
+      upload_work();
+      osteps = 0;
+    } else {
+      osteps++;
+    }
+    explicit_one_launch(otable.p, rwork.p, oblk.p, noblk, n, osteps, probes, stream);
+    pend_launches++;
   }
   void enqueue_resident() {
     const size_t tick_at = rwork_h.size() - 4 * sizeof(unsigned);
-    if (rwork.n < rwork_h.size()) rwork.alloc(2 * rwork_h.size());
-    NRT_HIP(hipMemcpyAsync(rwork.p, rwork_h.data(), rwork_h.size(), hipMemcpyHostToDevice, stream));
+    osteps = -1;
+    upload_work();
     for (int c = 0; c < 2; c++) {
       if (res[c].nwg == 0) continue;
       const int2* m = rmap.p + res[c].map_at;
@@ -364,7 +416,7 @@ struct nrt_batch {
         resident_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, res[c].lds,
                               stream);
       else
-        explicit_tree_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, rone, stream);
+        explicit_tree_batch_launch(rtable.p, rwork.p, m, ticket, res[c].nwg, res[c].T, stream);
       pend_launches++;
     }
   }
@@ -405,7 +457,7 @@ struct nrt_batch {
       launch_resident(k, elem_budget, kmax, cs, ss);
       // explicit slots take their steps together: those of the graph follow once no
       // exchange of these has timed out
-      if (!is_implicit() && !order.empty() && most > 1) {
+      if (!is_implicit() && !order.empty() && most > 1 && k > 1) {
         NRT_HIP(hipStreamSynchronize(stream));
         settle_exchanges();
       }

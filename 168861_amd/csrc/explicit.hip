@@ -30,10 +30,16 @@
 
 namespace nrt {
 
+// Where a step's gates go (the set they came from, or the other one).
+struct HHOut {
+  double *m, *h, *n;
+};
+__host__ __device__ __forceinline__ HHOut in_place(const HHDev& hd) { return HHOut{hd.m, hd.h, hd.n}; }
+
 // Forward-Euler HH gating of HH element i at potential v (solverEx-cpu.cpp:62-82,
 // coupling.cpp:25-48, discretization.cpp:81-86); returns W*dx and K*dx.
-__device__ __forceinline__ void hh_gate(const HHDev& hd, int i, double v, double dt_ms,
-                                        double& wdx, double& kdx) {
+__device__ __forceinline__ void hh_gate(const HHDev& hd, const HHOut& to, int i, double v,
+                                        double dt_ms, double& wdx, double& kdx) {
   const double rest = hd.rest[i];
   double vna = v + hd.ls_Na[i];
   double vk = v + hd.ls_K[i];
@@ -49,9 +55,9 @@ __device__ __forceinline__ void hh_gate(const HHDev& hd, int i, double v, double
   const double m = m0 + dt_ms * (am * (1 - m0) - bm * m0);
   const double h = h0 + dt_ms * (ah * (1 - h0) - bh * h0);
   const double n = n0 + dt_ms * (an * (1 - n0) - bn * n0);
-  hd.m[i] = m;
-  hd.h[i] = h;
-  hd.n[i] = n;
+  to.m[i] = m;
+  to.h[i] = h;
+  to.n[i] = n;
   const double gna = hd.g_Na[i] * m * m * m * h;
   const double gk = hd.g_K[i] * n * n * n * n;
   const double gl = hd.G_L[i];
@@ -143,7 +149,7 @@ template <bool NT, class VO, class VN>
 __device__ __forceinline__ void ex_finish_on(int j, const ExOps& o, VO Vo, VN Vn,
                                              const double* __restrict__ rdx_,
                                              const ExRec* __restrict__ recs_, const HHDev& hd,
-                                             double dt_ms, bool active) {
+                                             const HHOut& to, double dt_ms, bool active) {
   const NRT_GLB double* __restrict__ rdx = glb(rdx_);
   const uint32_t c = o.c, kind = c >> 29, idx = c & kCodeIdx;
   const double v = o.v;
@@ -152,7 +158,7 @@ __device__ __forceinline__ void ex_finish_on(int j, const ExOps& o, VO Vo, VN Vn
     // but an HH terminal still advances its gates (solverEx-cpu.cpp:62).
     if (kind == kExSkipHH) {
       double wd, kd;
-      hh_gate(hd, (int)idx, v, dt_ms, wd, kd);
+      hh_gate(hd, to, (int)idx, v, dt_ms, wd, kd);
     }
     return;
   }
@@ -162,7 +168,7 @@ __device__ __forceinline__ void ex_finish_on(int j, const ExOps& o, VO Vo, VN Vn
     // the sealed end right after it. One load waits on the code at most, none on
     // a record; the operations are the record path's, in its order.
     double wd = o.w0, kd = o.k0;
-    if (kind == kExHH) hh_gate(hd, (int)idx, v, dt_ms, wd, kd);
+    if (kind == kExHH) hh_gate(hd, to, (int)idx, v, dt_ms, wd, kd);
     const double vm = kind == kExDaughter ? Vo[idx] : o.vm;
     // (DL term +) DR term + mother term + W*dX*V + K*dX
     double s = (o.vp - v) / o.rp;
@@ -180,7 +186,7 @@ __device__ __forceinline__ void ex_finish_on(int j, const ExOps& o, VO Vo, VN Vn
   const int mo = rec.mother, dr = rec.dr, hh = rec.hh, fl = rec.flags;
   const int dl = (fl & 1) ? rec.dl : -1;
   double wd = o.w0, kd = o.k0;
-  if (hh >= 0) hh_gate(hd, hh, v, dt_ms, wd, kd);
+  if (hh >= 0) hh_gate(hd, to, hh, v, dt_ms, wd, kd);
   // branching*(DL term) + DR term + mother term + W*dX*V + K*dX + input
   const double tdr = (Vo[dr] - v) / rdx[dr];
   double s = (dl >= 0) ? ((Vo[dl] - v) / rdx[dl] + tdr) : tdr;
@@ -199,10 +205,10 @@ __device__ __forceinline__ void ex_finish(int j, const ExOps& o, const double* _
                                           double* __restrict__ Vn_,
                                           const double* __restrict__ rdx_,
                                           const ExRec* __restrict__ recs_, const HHDev& hd,
-                                          double dt_ms, bool active) {
+                                          const HHOut& to, double dt_ms, bool active) {
   const NRT_GLB double* __restrict__ Vo = glb(Vo_);
   NRT_GLB double* __restrict__ Vn = glb(Vn_);
-  ex_finish_on<true>(j, o, Vo, Vn, rdx_, recs_, hd, dt_ms, active);
+  ex_finish_on<true>(j, o, Vo, Vn, rdx_, recs_, hd, to, dt_ms, active);
 }
 
 __device__ __forceinline__ void explicit_element(
@@ -213,7 +219,7 @@ __device__ __forceinline__ void explicit_element(
     double dt_ms, bool active) {
   const ExOps o = ex_load(j, N, Vo, coefA, rdx, wdx, kdx, code);
   ex_ready(o);
-  ex_finish(j, o, Vo, Vn, rdx, recs, hd, dt_ms, active);
+  ex_finish(j, o, Vo, Vn, rdx, recs, hd, in_place(hd), dt_ms, active);
 }
 
 // One explicit step for every element (thread per element).
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(kResBlock) void k_explicit_resident(
     for (int j = tid; j < N; j += nt) {
       const ExOps o = ex_load_on(j, N, (const LdsD*)A, coefA, rdx, wdx, kdx, code);
       ex_ready(o);
-      ex_finish_on<false>(j, o, (const LdsD*)A, B, rdx, recs, hd, dt_ms, active);
+      ex_finish_on<false>(j, o, (const LdsD*)A, B, rdx, recs, hd, in_place(hd), dt_ms, active);
     }
     __syncthreads();
     LdsD* t = A;
@@ -579,7 +585,7 @@ __global__ __launch_bounds__(256) void k_explicit_batch(const ExSlot* __restrict
 #pragma unroll
   for (int u = 0; u < kExEPT; u++) {
     const int j = j0 + u * 256;
-    if (j < N) ex_finish(j, o[u], Vo, Vn, rdx, recs, S.hd, S.dt_ms, active);
+    if (j < N) ex_finish(j, o[u], Vo, Vn, rdx, recs, S.hd, in_place(S.hd), S.dt_ms, active);
   }
 }
 
@@ -632,6 +638,86 @@ void explicit_batch_steps(const void* slots, const int2* blk, int nblk, int nslo
   if (nslots > 0 && k > 0)
     hipLaunchKernelGGL(k_explicit_batch_trace, dim3(grid_for(nslots, 256)), dim3(256), 0, s, S,
                        nslots, gbase, k);
+  NRT_HIP(hipGetLastError());
+}
+
+// One step of slots that otherwise keep their elements in registers (explicit_tree.hip): over
+// memory, from one set of potentials and gates to the other as their launches go. What bounds
+// it is memory: 11 M elements 114 us, 5.1 TB/s. A call of one step in us, by that launch, by
+// a graph of one step before it, and so: 16 trees 24, 42, 18; 512 trees (5.5 M elements)
+// 94, 86, 72; 2,048 trees 325, 254, 252. Two steps are faster from registers (512 trees 94).
+struct ExOneSlot {
+  ExSlot s;
+  HHDev hd[2];  // the gates' sets, from either to the other
+  HHOut to[2];
+};
+__global__ __launch_bounds__(256) void k_explicit_batch_one(const ExOneSlot* __restrict__ slots,
+                                                            const ExTreeWork* __restrict__ work,
+                                                            const int2* __restrict__ blk, int i) {
+  const int2 b = blk[blockIdx.x];
+  const ExSlot& S = slots[b.x].s;
+  // (scalar loads together before the exit test, as in k_explicit_batch; the gates' places
+  // only where there are any)
+  const long long done = work[b.x].done + i, nst = S.num_steps, a0 = S.a0, a1 = S.a1;
+  const int cur = (work[b.x].cur + i) & 1, N = S.N;
+  const double* V0 = S.V[0];
+  const double* V1 = S.V[1];
+  const double* coefA = S.coefA;
+  const double* rdx = S.rdx;
+  const double* wdx = S.wdx;
+  const double* kdx = S.kdx;
+  const uint32_t* code = S.code;
+  const ExRec* recs = S.recs;
+  ready_s(V0);
+  ready_s(V1);
+  ready_s(coefA);
+  ready_s(rdx);
+  ready_s(wdx);
+  ready_s(kdx);
+  ready_s(code);
+  ready_s(recs);
+  const int j = b.y + (int)threadIdx.x;
+  if ((done >= nst) | (j >= N)) return;
+  const double* Vo = cur ? V1 : V0;
+  double* Vn = cur ? (double*)V0 : (double*)V1;
+  const ExOps o = ex_load(j, N, Vo, coefA, rdx, wdx, kdx, code);
+  ex_ready(o);
+  ex_finish(j, o, Vo, Vn, rdx, recs, slots[b.x].hd[cur], slots[b.x].to[cur], S.dt_ms,
+            done + 1 >= a0 && done + 1 <= a1);
+}
+// The probes that are due after it.
+__global__ void k_explicit_batch_one_trace(const ExOneSlot* __restrict__ slots,
+                                           const ExTreeWork* __restrict__ work, int n, int i) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const ExSlot& S = slots[k].s;
+  const long long after = work[k].done + i + 1;
+  if (after > S.num_steps || S.interval < 0 || !S.trace || after % (S.interval + 1) != 0) return;
+  S.trace[after / (S.interval + 1) - 1] = S.V[(work[k].cur + i + 1) & 1][S.trace_elem];
+}
+
+size_t explicit_one_bytes() { return sizeof(ExOneSlot); }
+void explicit_one_fill(nrt_handle* h, long long num_steps, long long a0, long long a1,
+                       int trace_elem, long long interval, double* trace, void* out) {
+  Explicit* e = h->ex;
+  ExOneSlot S{};
+  explicit_slot_fill(h, 0, num_steps, a0, a1, trace_elem, interval, trace, &S.s);
+  S.hd[0] = S.hd[1] = e->hd();
+  S.hd[1].m = e->m2.p;
+  S.hd[1].h = e->h2.p;
+  S.hd[1].n = e->n2.p;
+  S.to[0] = in_place(S.hd[1]);
+  S.to[1] = in_place(S.hd[0]);
+  std::memcpy(out, &S, sizeof(S));
+}
+// The i-th step after the one that `work` was made for.
+void explicit_one_launch(const void* slots, const void* work, const int2* blk, int nblk,
+                         int nslots, int i, bool probes, hipStream_t s) {
+  hipLaunchKernelGGL(k_explicit_batch_one, dim3(nblk), dim3(256), 0, s, (const ExOneSlot*)slots,
+                     (const ExTreeWork*)work, blk, i);
+  if (probes)
+    hipLaunchKernelGGL(k_explicit_batch_one_trace, dim3(grid_for(nslots, 256)), dim3(256), 0, s,
+                       (const ExOneSlot*)slots, (const ExTreeWork*)work, nslots, i);
   NRT_HIP(hipGetLastError());
 }
 

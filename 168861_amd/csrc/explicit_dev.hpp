@@ -119,6 +119,14 @@ __device__ __forceinline__ bool ex_get(const ExWord* w, unsigned tag, int nv,
   return true;
 }
 
+// A batch slot's work in a launch (explicit_tree.hip): steps done before it and taken by it,
+// the set that holds potentials and gates before it, exchanges so far.
+struct ExTreeWork {
+  long long done, steps;
+  int cur;
+  unsigned tag;
+};
+
 // explicit_cable.hip
 // A launch whose G workgroups exchange values, until it ends without a time-out:
 // launch(polls of the first exchange, of the others).

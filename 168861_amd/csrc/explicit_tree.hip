@@ -81,8 +81,6 @@ __device__ __forceinline__ void ex_load8(const __attribute__((address_space(1)))
   }
 }
 
-// ONE: a single step, which no exchange comes into; halo units only show their potentials.
-template <bool ONE>
 __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRun& q, int g) {
   constexpr int C = kExC;
   __shared__ double val[2][kExVals];
@@ -110,7 +108,7 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
   unsigned tag = q.tag0;
   int p = 0, left = every;
   unsigned long long most = q.first_limit;
-  const long long first = pinned_s(q.first), end = ONE ? first + 1 : pinned_s(first + q.num);
+  const long long first = pinned_s(q.first), end = pinned_s(first + q.num);
   // a step's sample is due: advances the count
   auto sample = [&]() {
     if (interval < 0 || ++gl <= interval) return false;
@@ -128,10 +126,7 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
     // (an unused place reads what lies before the unit, or, at the arrays' beginning, the
     // unit's first element: no load waits for another)
     const int at = u.first - f;
-    const bool shows = ONE && halo;
-    if (shows && at >= 0) {
-      ex_load8(Vin + at, V);
-    } else if (on && at >= 0) {
+    if (on && at >= 0) {
       ex_load8(Vin + at, V);
       ex_load8(coefA + at, a);
       ex_load8(rdx + at, r);
@@ -152,14 +147,13 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
     for (int k = 0; k < C; k++) {
       const bool used = k >= f;
       V[k] = used ? V[k] : 0.0;
-      a[k] = used && !shows ? a[k] : 0.0;
-      r[k] = used && !shows ? r[k] : 1.0;
-      w[k] = used && !shows ? w[k] : 0.0;
-      kd[k] = used && !shows ? kd[k] : 0.0;
+      a[k] = used ? a[k] : 0.0;
+      r[k] = used ? r[k] : 1.0;
+      w[k] = used ? w[k] : 0.0;
+      kd[k] = used ? kd[k] : 0.0;
       y[k] = 1 / r[k];
     }
-    const double rR = on && !shows ? rdx[u.el_right] : 1.0,
-                 rL = on && !shows ? rdx[u.el_left] : 1.0;
+    const double rR = on ? rdx[u.el_right] : 1.0, rL = on ? rdx[u.el_left] : 1.0;
     const double yR = 1 / rR, yL = 1 / rL;
     double v0 = ghost ? Vin[0] : 0.0;
     const int up = on ? u.up : kExMissing, right = on && !term ? u.right : kExMissing;
@@ -188,7 +182,7 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
     publish();
     lds_sync();
     for (long long i = first; i < end; i++) {
-      if (!ONE && left == 0) {
+      if (left == 0) {
         left = every;
         tag++;
         const bool has = on && u.slot >= 0;
@@ -313,7 +307,7 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
     if (e == 0) val[p][at] = v;
     lds_sync();
     for (long long i = first; i < end; i++) {
-      if (!ONE && left == 0) {
+      if (left == 0) {
         left = every;
         tag++;
         const bool has = on && u.slot >= 0;
@@ -384,7 +378,7 @@ __device__ __forceinline__ void ex_tree_steps(const ExTreeDev& d, const ExTreeRu
 }
 
 __global__ __launch_bounds__(kExTBlock) void k_explicit_tree(ExTreeDev d, ExTreeRun q) {
-  ex_tree_steps<false>(d, q, (int)blockIdx.x);
+  ex_tree_steps(d, q, (int)blockIdx.x);
 }
 
 // Slots of a batch: workgroup w of the launch order runs map[w] = (slot, group) for the
@@ -393,11 +387,6 @@ __global__ __launch_bounds__(kExTBlock) void k_explicit_tree(ExTreeDev d, ExTree
 struct ExTreeRec {
   ExTreeDev d;
   double* trace_base;
-};
-struct ExTreeWork {
-  long long done, steps;
-  int cur;
-  unsigned tag;
 };
 __global__ __launch_bounds__(kExTBatch + kWave) void k_explicit_tree_batch(
     const ExTreeRec* __restrict__ recs, const ExTreeWork* __restrict__ work,
@@ -413,26 +402,7 @@ __global__ __launch_bounds__(kExTBatch + kWave) void k_explicit_tree_batch(
     q.gl0 = wk.done % (rec.d.interval + 1);
     if (rec.trace_base) q.trace = rec.trace_base + wk.done / (rec.d.interval + 1);
   }
-  ex_tree_steps<false>(rec.d, q, m.y);
-}
-
-// One step of every slot: no workgroup waits for another, so any order does, and what counts
-// is how many waves have loads in flight: four a SIMD instead of three (512 trees, 5.5 M
-// elements: 74 us; 83 by the kernel above, 66 by a launch a step that goes over memory, but
-// 84, 94 and 85 with what a call costs besides).
-__global__ __launch_bounds__(kExTBatch + kWave, 4) void k_explicit_tree_batch_one(
-    const ExTreeRec* __restrict__ recs, const ExTreeWork* __restrict__ work,
-    const int2* __restrict__ map) {
-  const int2 m = map[blockIdx.x];
-  const ExTreeRec& rec = recs[m.x];
-  const ExTreeWork wk = work[m.x];
-  if (wk.steps < 1) return;
-  ExTreeRun q{wk.cur, wk.done + 1, 1, 0, nullptr, wk.tag, 0, 0};
-  if (rec.d.interval >= 0) {
-    q.gl0 = wk.done % (rec.d.interval + 1);
-    if (rec.trace_base) q.trace = rec.trace_base + wk.done / (rec.d.interval + 1);
-  }
-  ex_tree_steps<true>(rec.d, q, m.y);
+  ex_tree_steps(rec.d, q, m.y);
 }
 
 // ---------------------------------------------------------------- host side
@@ -609,13 +579,7 @@ void explicit_tree_undo(nrt_handle* h, const void* work, long long* done, long l
   *steps = w.steps;
 }
 void explicit_tree_batch_launch(const void* recs, const void* work, const int2* map,
-                                unsigned* ticket, int nwg, int T, bool one, hipStream_t s) {
-  if (one) {
-    hipLaunchKernelGGL(k_explicit_tree_batch_one, dim3(nwg), dim3(T + kWave), 0, s,
-                       (const ExTreeRec*)recs, (const ExTreeWork*)work, map);
-    NRT_HIP(hipGetLastError());
-    return;
-  }
+                                unsigned* ticket, int nwg, int T, hipStream_t s) {
   const char* sl = getenv("NRT_SPIN_LIMIT");
   hipLaunchKernelGGL(k_explicit_tree_batch, dim3(nwg), dim3(T + kWave), 0, s,
                      (const ExTreeRec*)recs, (const ExTreeWork*)work, map, ticket,
