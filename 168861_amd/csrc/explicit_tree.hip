@@ -513,11 +513,12 @@ static ExTreeDev tree_dev(Explicit* e, int from, unsigned* err, long long a0, lo
 int64_t tree_run(nrt_handle* hnd, Explicit* e, int64_t first, int64_t num, int64_t a0, int64_t a1,
                  int32_t trace_elem, int64_t interval, double* trace, hipEvent_t t0,
                  hipEvent_t t1) {
-  // One or two steps go over memory, as fast as the registers are filled and emptied (run
-  // of 1 / 2 / 4 steps there and here, us, with the launch and the wait: 700 elements 18 / 20
-  // / 25 and 23 / 24 / 25; 30,000 18 / 22 / 30 and 24 / 24 / 25; 902,037 23 / 33 / 53 and
-  // 30 / 32 / 33).
-  if (e->tree_groups == 0 || num <= 2) return 0;
+  // One or two steps, and three of a short neurite, are done without the registers, as fast as
+  // these are filled and emptied (run of 1 / 2 / 3 / 4 steps there and here, us, with the
+  // launch and the wait: 300 elements 18 / 21 / 23 / 25 and 23 / 24 / 24 / 25; 2,000
+  // 20 / 23 / 26 / 29 and 24 / 25 / 26 / 26; 30,000 18 / 22 / 27 / 30 and 24 / 24 / 25 / 25;
+  // 902,037 23 / 33 / 43 / 53 and 30 / 32 / 33 / 33).
+  if (e->tree_groups == 0 || num <= (e->N <= 1500 ? 3 : 2)) return 0;
   // (pieces: see run_persistent in implicit.hip; 8,192 steps of 902,037 elements 12 ms)
   constexpr int64_t kShareSteps = 8192;
   constexpr int kShareCus = 64;
