@@ -1,8 +1,9 @@
 // Batches of independent neurites (the nrt_batch_* entry points). Each slot is a
 // complete solver state (a handle without a stream of its own); the batch keeps a
 // device table of slot descriptors that is rebuilt only when membership changes,
-// and advances all slots with one launch per call (persistent over the k steps) or,
-// for explicit slots whose elements cannot stay in registers, one graph of k steps.
+// and advances all slots with one launch per call (persistent over the k steps; a single
+// explicit step goes over memory) or, for explicit slots whose elements cannot stay in
+// registers, one graph of k steps.
 #include <algorithm>
 #include <chrono>
 #include <climits>
@@ -84,7 +85,8 @@ inline int size_class(int N) { return N < 4096 ? 0 : (N < 16384 ? 1 : 2); }
 constexpr int kPlanThreads = 256;
 // Footprint per element used for admission (bytes; the arrays a slot allocates,
 // rounded up): implicit tree solve ~ 7 FP64 + 3 int32 vectors, 3 CSR entries, the
-// plan and 8 tree work values over ~1.1 N level nodes; explicit ~ 6 FP64 + code.
+// plan and 8 tree work values over ~1.1 N level nodes; explicit ~ 6 FP64 + code and 12 for
+// a plan (a larger one is made only while there is room, tree_room in explicit_tree.hip).
 constexpr int64_t kImplicitBytesPerElem = 420;
 constexpr int64_t kExplicitBytesPerElem = 64;
 constexpr int64_t kAdmissionReserve = 512ll << 20;  // left free for the runtime

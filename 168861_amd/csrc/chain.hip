@@ -1,5 +1,5 @@
 // Exact solve of an unbranched neurite (an axon with any number of Hodgkin-Huxley nodes
-// up to one row in eight) with its rows resident in registers: a wave per 64 kChC rows.
+// up to one row in eight) with its rows resident in registers: a wave per 64 C rows.
 //
 // The matrix is tridiagonal. Levels, each the same elimination with one row kept:
 //   lane  C rows: all but the last in terms of the last row of the lane before and its

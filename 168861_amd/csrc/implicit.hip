@@ -2068,8 +2068,8 @@ static int choose_blocks(nrt_handle* hnd, int N, const void* kernel = nullptr) {
 // The resident form (resident.hpp) of a FP64 direct solve, with every option that
 // shapes the other forms left to the library. Taken whenever its plan exists and a
 // launch's workgroups are all resident at once, whatever the size: per step, 700 rows
-// 30.4 us in block form, 2.7 resident; 3,001 rows 36.7 and 4.3; 60,000 rows (17 groups)
-// 49.7 (local form) and 9.5; 902,037 rows (255 groups) 120 and 14.0.
+// 30.4 us in block form, 2.6 resident; 3,001 rows 36.7 and 3.8; 60,000 rows (17 groups)
+// 49.7 (local form) and 8.8; 902,037 rows (253 groups) 120 and 12.8.
 static bool resident_create(nrt_handle* hnd, Implicit* e, const HostProblem& p,
                             const std::vector<int32_t>& par, const std::vector<int32_t>& rowptr,
                             const std::vector<int32_t>& col, const std::vector<double>& cmdx,

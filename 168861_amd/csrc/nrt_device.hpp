@@ -102,7 +102,9 @@ __device__ __forceinline__ double rcp_newton(double x) {
 }
 
 // x / c from y = 1 / c (rounded): the quotient's first estimate, its exact remainder,
-// one correction; infinite x as a division takes it.
+// one correction; infinite x as a division takes it. Rounds as the division does where
+// |x| and the quotient are above 2^-968 (the remainder is exact) and the quotient does not
+// overflow (it would be NaN); below, it may be off by the last bit.
 __device__ __forceinline__ double div_by(double x, double c, double y) {
   const double q = x * y;
   return __builtin_amdgcn_div_fixup(fma(fma(-c, q, x), y, q), c, x);

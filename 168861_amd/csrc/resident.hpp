@@ -58,7 +58,8 @@ struct ResPlanHost {
   std::vector<double> F, I;        // [G * C * T]
   std::vector<double> uco;         // kUnitArrays x [G * T]
   std::vector<uint32_t> uinf;      // 3 words per unit: piece | pos << 10 | len << 16 |
-                                   // top << 31; na | pa << 16; sa | parent piece << 16
+                                   // top << 31; na | pa << 16; the strand's own top node
+                                   // (nt: none) | parent piece << 16
   std::vector<double> pz;          // [G * T] Z of each piece
   std::vector<uint16_t> pinf;      // 8 per piece: child pieces, parent piece, height,
                                    // published o, published x, 0, 0

@@ -281,7 +281,10 @@ int nrt_destroy(nrt_handle* h);                       /* Solver::~Solver   */
  * active_first <= i <= active_last; every trace_every steps (counting as the
  * reference's GL_cont) V[trace_elem] is recorded into trace_out.
  * trace_out may be NULL when trace_every <= 0. Returns the number of samples in
- * *num_samples.
+ * *num_samples. A long run that takes most of the device is several launches
+ * (nrt_stats.kernel_launches); one that ends with NRT_ERR_HIP because another
+ * process held part of the device leaves the state after those that ended
+ * (nrt_stats.steps counts them).
  */
 int nrt_run(nrt_handle* h, int64_t first_step, int64_t num_steps,
             int64_t active_first, int64_t active_last,
@@ -302,9 +305,12 @@ int nrt_sync(nrt_handle* h);
  *     of their own, concurrently, while every class fills at least half the
  *     device, else all in one launch;
  *   explicit: the k steps of a call in one launch with every element in registers
- *     (at most eight HH elements on a tree or cable); other slots one thread per
- *     element, one launch per step, the k steps captured once as a HIP graph and
- *     replayed.
+ *     (at most eight HH elements on a tree or cable; very many steps in several
+ *     launches, a single one over memory); other slots one thread per element, one
+ *     launch per step, the k steps captured once as a HIP graph and replayed. A call
+ *     that fails with NRT_ERR_HIP because another process held part of the device
+ *     leaves every slot after the same number of its steps (none, unless the message
+ *     says how many).
  * Slots keep their whole state on the device and join or leave between calls
  * (continuous batching). A slot counts its own steps from 1: its stimulus is on
  * for steps a0..a1 and it completes after num_steps. Probe traces follow
